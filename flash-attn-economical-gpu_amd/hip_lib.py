@@ -122,6 +122,15 @@ SIGNATURES = {
             ctypes.POINTER(GemmTile), ctypes.c_void_p,
         ],
     ),
+    "gemm_f16_ldb4": (
+        ctypes.c_int,
+        [
+            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+            ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+            ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+            ctypes.POINTER(GemmTile), ctypes.c_void_p,
+        ],
+    ),
     "gemm_f16_supported": (ctypes.c_int, [ctypes.POINTER(GemmTile)]),
     "fa_kernel_resources": (
         ctypes.c_int,
@@ -318,8 +327,9 @@ def fa_fwd_noalloc(
     check(lib.fa_fwd_noalloc(ctypes.byref(args), _stream_ptr(q.device)), "fa_fwd_noalloc")
 
 
-def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile) -> None:
-    """C = A @ B (fp16, fp32 accumulation) written into c on the current stream."""
+def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile, *, ldb4: bool = False) -> None:
+    """C = A @ B (fp16, fp32 accumulation) written into c on the current stream. ldb4: B's row pitch is
+    only a multiple of 4 elements (the gemm_f16_ldb4 entry)."""
     lib = load()
     for name, t in (("a", a), ("b", b), ("c", c)):
         if t.dim() != 2 or t.device.type != "cuda" or t.dtype != torch.float16:
@@ -330,7 +340,7 @@ def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile) 
     K2, N = b.shape
     if K2 != K or tuple(c.shape) != (M, N):
         raise ValueError(f"incompatible GEMM shapes a={tuple(a.shape)} b={tuple(b.shape)} c={tuple(c.shape)}")
-    code = lib.gemm_f16(
+    code = (lib.gemm_f16_ldb4 if ldb4 else lib.gemm_f16)(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K,
         a.stride(0), b.stride(0), c.stride(0), ctypes.byref(tile), _stream_ptr(a.device),
     )

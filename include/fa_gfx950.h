@@ -190,6 +190,11 @@ int fa_fwd_supported(int32_t variant, int32_t dtype, int32_t D, const fa_tile* t
 int gemm_f16(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K,
              int64_t lda, int64_t ldb, int64_t ldc, const gemm_tile* tile, void* stream);
 
+/* gemm_f16 for a B whose rows start on 8-byte boundaries only (ldb a multiple of 4; the base pointer
+ * 16-byte aligned as for gemm_f16). No counterpart in the reference, which needs N % 64 == 0. */
+int gemm_f16_ldb4(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K,
+                  int64_t lda, int64_t ldb, int64_t ldc, const gemm_tile* tile, void* stream);
+
 int gemm_f16_supported(const gemm_tile* tile);
 
 /* Resources of one built kernel: op 0 = attention (variant, dtype, D, tile; the kernel that tile

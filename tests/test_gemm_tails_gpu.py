@@ -61,7 +61,7 @@ def test_gemm_tails_all_tiles(gpu, shape):
                          ids=["n_mod8_0", "n_mod8_4", "n_mod8_4_deep"])
 def test_gemm_tails_convenience_entry(gpu, shape):
     """mma.matmul takes tail shapes (the reference selector still raises for them), N % 8 == 4
-    included (B is restaged into rows of a multiple of 8 elements)."""
+    included (B is read in place, its rows on 8-byte boundaries)."""
     M, N, K = shape
     print(f"[gemm_tails] mma.matmul {M}x{N}x{K}", flush=True)
     with pytest.raises(ValueError):
@@ -74,6 +74,40 @@ def test_gemm_tails_convenience_entry(gpu, shape):
     ref = oracle.gemm(a, b)
     assert float(np.linalg.norm(c.float().cpu().numpy() - ref) / np.linalg.norm(ref)) <= 1e-3
     assert cfgs.choose_gemm_tile_any(M, N, K)[:3] != ()
+
+
+@pytest.mark.parametrize("pad", [0, 8], ids=["tight", "padded"])
+@pytest.mark.parametrize("shape", [(33, 4, 8), (65, 60, 520), (260, 396, 264), (1000, 1004, 1000)],
+                         ids=["33x4x8", "65x60x520", "260x396x264", "1000x1004x1000"])
+def test_gemm_rows_of_b_on_8_byte_boundaries(gpu, shape, pad):
+    """B rows whose pitch is 4 mod 8 elements, read in place: every other row starts 8 bytes past a
+    16-byte boundary and the last row's last 16-byte piece crosses the end of the buffer range. NaN past
+    N (padded) or in the next row's place after the last row must not reach C."""
+    M, N, K = shape
+    print(f"[gemm_tails] ldb4 M={M} N={N} K={K} pad={pad}", flush=True)
+    a = oracle.round_to(oracle.portable_uniform(41, (M, K), -1, 1), 0)
+    b = oracle.round_to(oracle.portable_uniform(42, (K, N), -1, 1), 0)
+    ref = oracle.gemm(a, b)
+    ad = to_device(a, torch.float16, "cuda:0")
+    ldb = N + pad
+    bbuf = torch.full((K + 1, ldb), float("nan"), dtype=torch.float16, device="cuda:0")
+    bd = bbuf[:K, :N]
+    bd.copy_(to_device(b, torch.float16, "cuda:0"))
+    for tile in TILES:
+        cd = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda:0")
+        hip_lib.gemm_f16(ad, bd, cd, hip_lib.GemmTile(*tile, 4), ldb4=True)
+        torch.cuda.synchronize()
+        c = cd.float().cpu().numpy()
+        assert np.isfinite(c).all(), tile
+        # fp32 sums and one rounding to binary16: 2^-12 relative per element, the bound of the other tests
+        assert float(np.linalg.norm(c - ref) / np.linalg.norm(ref)) <= 1e-3, tile
+    with pytest.raises(ValueError, match="leading dimensions"):
+        hip_lib.gemm_f16(ad, bd, cd, hip_lib.GemmTile(*TILES[0], 4))  # gemm_f16 keeps its 16-byte rows
+    if pad == 0:  # a B whose base is not 16-byte aligned is restaged
+        flat = torch.empty(K * N + 4, dtype=torch.float16, device="cuda:0")
+        shifted = flat[4:].view(K, N)
+        shifted.copy_(bd)
+        torch.testing.assert_close(mma.matmul(ad, shifted), mma.matmul(ad, bd.contiguous()), rtol=0, atol=0)
 
 
 def test_gemm_rejects_unaligned_tails(gpu):
