@@ -267,6 +267,22 @@ def test_fa_persistent_items(gpu, case):
     assert max_abs(lse9.reshape(-1)[rows], lse_ref) <= 1e-3, name
 
 
+@pytest.mark.parametrize("stages", [8, 9])
+@pytest.mark.parametrize("M,N,causal,splits", [(256, 704, False, 1), (300, 1000, False, 3), (700, 700, True, 1),
+                                               (700, 900, True, 4), (513, 1025, True, 2), (1100, 1100, True, 1)])
+def test_fa_ping_pong_masked_range(gpu, stages, M, N, causal, splits):
+    """The ping-pong kernels run their unmasked inner steps in a loop of their own, up to the first
+    tile that needs a mask: ranges where that tile is the last, inside, before the split's first tile,
+    or different for the waves of a workgroup."""
+    q, k, v = make_qkv(77 + M + N, 2, 3, 3, M, N, 128, BF16)
+    print(f"[fa_abi] masked range stages={stages} M={M} N={N} causal={causal} splits={splits}", flush=True)
+    variant = SLICED if splits > 1 else OPT
+    o, lse = run_fa(q, k, v, variant=variant, tile=(variant, 256, 64, 8, stages), causal=causal, dtype=BF16, splits=splits)
+    o_ref, lse_ref = oracle.attention(q, k, v, causal=causal)
+    assert max_abs(o, o_ref) <= ATOL[BF16]
+    assert max_abs(lse, lse_ref) <= 1e-3
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_fa_parity(gpu, case):
     name, B, H, Hkv, M, N, D, dtype, causal, tile_name = case
