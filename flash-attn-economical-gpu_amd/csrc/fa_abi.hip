@@ -45,7 +45,7 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 const fa::FaKernelEntry* find_fwd(int stages, int dtype, int D, int waves, int rows_per_wave, int block_n,
                                   int split) {
-  // stages 1-5: fa_fwd.hip (32x32x16 MFMAs); stages 6-9: fa_fwd16.hip (16x16x32 MFMAs)
+  // stages 1-5: fa_fwd.hip (32x32x16 MFMAs); stages 6-10: fa_fwd16.hip (16x16x32 MFMAs)
   int n = 0;
   const fa::FaKernelEntry* e = stages >= 6 ? fa::fa_fwd16_registry(&n) : fa::fa_fwd_registry(&n);
   for (int i = 0; i < n; ++i)
@@ -74,10 +74,11 @@ const fa::GemmKernelEntry* find_gemm(const gemm_tile* t) {
 }
 
 // Pipeline of a launch: basic keeps one K/V buffer (1); optimized and sliced double-buffer K/V (2),
-// or, when the tile asks for stages 3-9, run that LDS-DMA kernel (3-5: 32x32x16 MFMA tiles, 6-9:
-// 16x16x32 ones; the stages doc of fa_tile in the header lists them).
+// or, when the tile asks for stages 3-10, run that LDS-DMA kernel (3-5: 32x32x16 MFMA tiles, 6-10:
+// 16x16x32 ones; the stages doc of fa_tile in the header lists them; 10 is built for one tile only).
 int stages_of(int variant, const fa_tile* t) {
   if (variant == FA_VARIANT_BASIC) return 1;
+  if (t != nullptr && t->stages == 10 && t->waves == 8 && t->block_m == 128) return 10;
   return (t != nullptr && t->stages >= 3 && t->stages <= 9) ? t->stages : 2;
 }
 
@@ -152,6 +153,8 @@ bool pipelined_fits(const fa_fwd_args* a, int block_n) {
 // The double-buffered kernel that replaces a pipelined one when pipelined_fits() fails: same
 // dtype, D, waves, rows per wave and split, the same block_n if built, else 64 keys.
 const fa::FaKernelEntry* double_buffered_fallback(const fa::FaKernelEntry* e) {
+  // the key-group kernel's 8 waves share 128 rows: 4 waves of 32 rows replace them
+  if (e->stages == 10) return find_fwd(2, e->dtype, e->D, 4, 32, e->block_n, e->split);
   const fa::FaKernelEntry* fb = find_fwd(2, e->dtype, e->D, e->waves, e->rows_per_wave, e->block_n, e->split);
   if (fb == nullptr) fb = find_fwd(2, e->dtype, e->D, e->waves, e->rows_per_wave, 64, e->split);
   return fb;
@@ -259,7 +262,7 @@ static int launch_fwd(const fa_fwd_args* a, void* ws, int64_t ws_bytes, void* st
   if (!std::isfinite(a->sm_scale) || a->sm_scale <= 0.f)
     return fail(FA_EINVAL, "sm_scale must be positive and finite, got %g", (double)a->sm_scale);
 
-  if (e->stages >= 3 && !pipelined_fits(a, e->block_n)) {
+  if (e->stages >= 3 && !pipelined_fits(a, e->stages == 10 ? 2 * e->block_n : e->block_n)) {
     // The pipelined kernel addresses one (batch, kv-head) row range [0, N + block_n) of K and V
     // with 32-bit byte offsets and relies on whole rows for its tail check: run the
     // double-buffered kernel of the same rows per workgroup instead (same block_n where it is

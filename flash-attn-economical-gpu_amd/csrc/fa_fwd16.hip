@@ -35,7 +35,8 @@ struct Fwd16 {
   static constexpr int THREADS = WAVES * 64;
   static constexpr int QT = 2;            // 16-query tiles per wave
   static constexpr int ROWS = 16 * QT;    // query rows per wave
-  static constexpr int BM = WAVES * ROWS;
+  static constexpr int KG = PIPE == 4 ? 2 : 1;  // groups of waves that share the rows and split the keys
+  static constexpr int BM = WAVES / KG * ROWS;
   static constexpr int DC = D / 32;       // 32-deep d chunks of Q K^T
   static constexpr int DTL = D / 16;      // 16-row d tiles of O^T
   static constexpr int JT = BN / 16;      // 16-key score tiles
@@ -131,11 +132,14 @@ struct Fwd16 {
   // sign-bit mask and a bitfield select -- vector ALU only: per-element compares would each hold a
   // scalar register pair, and the scheduler hoists all 32 of them.
   __device__ static inline void mask_tile(STile& s, int n0, int wrow0, int q16, int g, const FwdParams& p) {
+    mask_tile(s, n0, wrow0, q16, g, p.N, p.causal != 0);
+  }
+  __device__ static inline void mask_tile(STile& s, int n0, int wrow0, int q16, int g, int n_lim, bool causal) {
     const uint32_t ninf = __float_as_uint(FA_NEG_INF);
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
       const int i = wrow0 + qt * 16 + q16;
-      const int lim = p.causal ? min(p.N, i + 1) : p.N;
+      const int lim = causal ? min(n_lim, i + 1) : n_lim;
 #pragma unroll
       for (int jt = 0; jt < JT; ++jt) {
         const int rel = lim - (n0 + jt * 16 + 4 * g);  // keys r < rel of this lane are kept
@@ -247,6 +251,15 @@ struct Fwd16 {
     tile_max(s, mx);
     rescale(mx, acc, ro, l_i, lsum, p.c);
     exp_pack(s, pk, ro, l_i, p.c);
+  }
+
+  // The same for a tile that needs no mask.
+  __device__ static inline void softmax_unmasked(const STile& s, u32x4 (&pk)[KC][QT], OAcc& acc, RowOff& ro,
+                                                 float (&l_i)[QT], floatx4 (&lsum)[QT], float c) {
+    float mx[QT];
+    tile_max(s, mx);
+    rescale(mx, acc, ro, l_i, lsum, c);
+    exp_pack(s, pk, ro, l_i, c);
   }
 
   // P = exp2(S c - m c) rounded to the input dtype and packed as the B operand of P V; the row
@@ -1111,6 +1124,282 @@ struct Fwd16 {
     }
   }
 
+  // ---- key groups (stages=10) ---------------------------------------------------------------------
+  // The ping-pong schedule for grids too small to fill the chip with 256-row blocks: a block is 128
+  // query rows, and its two groups of four waves hold the same rows and take alternate KV tiles
+  // (group 0 tiles 0, 2, ..., group 1 tiles 1, 3, ...), one phase apart as in run(). Twice the blocks
+  // with half the serial steps each, at twice the K/V fetch per step (a ring slot holds a pair of
+  // tiles); the two partial results meet through LDS at the end, so there is no workspace and no
+  // second launch. What bounds the small grids it is for is the longest block's chain of steps: bf16
+  // B1 H12/2 D128 causal N=4096 94 -> 70 us (740 TFLOP/s), B2 H16 D64 777x1283 26 -> 19, fp16 B1 H28
+  // D128 N=1024 29 -> 22. A step costs 1.35 ping-pong steps, so grids that fill the chip stay there.
+  __device__ static void run_key_groups(const FwdParams& p) {
+    static_assert(PIPE != 4 || (WAVES == 8 && BN == 64 && KG == 2), "two groups of four waves");
+    constexpr uint32_t kPairK = 2 * KT_ELEMS * 2, kPairV = 2 * VT_ELEMS * 2;  // bytes of a ring slot
+    __shared__ __attribute__((aligned(16))) uint16_t smem[4 * (KT_ELEMS + VT_ELEMS)];
+    const int tid = (int)__builtin_amdgcn_workitem_id_x();
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q16 = lane & 15, g = lane >> 4;
+
+    // Causal: heaviest query blocks of all heads first, heads fastest (with a multiple of 8 heads a
+    // head's blocks stay on one XCD), so the last blocks to start are the short ones. Otherwise
+    // neighbouring blocks of a head on one XCD, as run().
+    int mb, rest;
+    const int wg = (int)__builtin_amdgcn_workgroup_id_x();
+    if (p.causal) {
+      const int heads = p.total_blocks / p.m_blocks;
+      mb = p.m_blocks - 1 - wg / heads;
+      rest = wg % heads;
+    } else {
+      const int pid = xcd_remap(wg, p.total_blocks);
+      mb = pid % p.m_blocks;
+      rest = pid / p.m_blocks;
+    }
+    mb = __builtin_amdgcn_readfirstlane(mb);
+    const int split = __builtin_amdgcn_readfirstlane(rest % p.splits);
+    const int bh = rest / p.splits;
+    const int bheads = p.pack > 1 ? p.Hkv : p.H;
+    const int b = __builtin_amdgcn_readfirstlane(bh / bheads);
+    const int hi = bh % bheads;
+    const int h = __builtin_amdgcn_readfirstlane(p.pack > 1 ? hi * p.group : hi);
+    const int hk = __builtin_amdgcn_readfirstlane(h / p.group);
+    const int rows = p.M * p.pack;
+    const int m0 = mb * BM;
+    const int wrow0 = m0 + (wave & 3) * ROWS;
+    const bool wave_has_rows = wrow0 < rows;
+
+    u32x4 qf[QT][DC];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const int row = wrow0 + qt * 16 + q16;
+      const int hr = p.pack > 1 ? h + row / p.M : h, mr = p.pack > 1 ? row % p.M : row;
+      const uint16_t* qrow = p.q + (int64_t)b * p.sq0 + (int64_t)hr * p.sq1 + (int64_t)mr * p.sq2;
+#pragma unroll
+      for (int cc = 0; cc < DC; ++cc) {
+        u32x4 val = {0u, 0u, 0u, 0u};
+        if (row < rows) val = *reinterpret_cast<const u32x4*>(qrow + cc * 32 + g * 8);
+        qf[qt][cc] = val;
+      }
+    }
+
+    const int t_begin = split * p.tiles_per_split;
+    int n_end = min((t_begin + p.tiles_per_split) * BN, p.N);
+    if (p.causal) n_end = min(n_end, m0 + BM);
+    n_end = __builtin_amdgcn_readfirstlane(n_end);
+    const int ntiles = max((n_end + BN - 1) / BN - t_begin, 0);
+    const int nsteps = (ntiles + 1) / 2;
+
+    OAcc acc;
+    RowOff ro;
+    ro.reset();
+    float l_i[QT];
+    floatx4 lsum[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      l_i[qt] = 0.f;
+      lsum[qt] = (floatx4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int dt = 0; dt < DTL; ++dt) acc[dt][qt] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    }
+
+    // DMA sources and ring as run(); a slot holds the K (V) tiles of both groups. Keys past N read
+    // zeros; keys of a pair's second tile past the range's end are masked.
+    const u32x4 krs = make_rsrc(p.k + (int64_t)b * p.sk0 + (int64_t)hk * p.sk1, (uint32_t)p.N * (uint32_t)p.sk2 * 2u);
+    const u32x4 vrs = make_rsrc(p.v + (int64_t)b * p.sv0 + (int64_t)hk * p.sv1, (uint32_t)p.N * (uint32_t)p.sv2 * 2u);
+    uint32_t koff, voff;
+    {
+      const int blk = wave * NKW, jt = blk / DC, cc = blk % DC;
+      koff = ((uint32_t)(jt * 16 + q16) * (uint32_t)p.sk2 + cc * 32 + 8 * g) * 2u;
+    }
+    {
+      const int blk = wave * NVW, kc = blk / DTL, dt = blk % DTL;
+      const uint32_t row = kc * 32 + 16 * (lane >> 5) + 4 * ((lane & 31) >> 3) + ((lane & 7) >> 1);
+      voff = (row * (uint32_t)p.sv2 + dt * 16 + 8 * (lane & 1)) * 2u;
+    }
+    const uint32_t kring_lds = lds_address(smem), vring_lds = kring_lds + 2 * kPairK;
+    const uint32_t ktile = (uint32_t)BN * (uint32_t)p.sk2 * 2u, vtile = (uint32_t)BN * (uint32_t)p.sv2 * 2u;
+    // A tile that starts past N has no valid byte: its resource gets range 0 (slab_rsrc needs an
+    // offset within the range).
+    auto issue_k = [&](int u) __attribute__((always_inline)) {
+      if (u >= nsteps) return;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int t = t_begin + 2 * u + x;
+        const bool live = t * BN < p.N;
+        buffer_load16_to_lds_blocks<NKW, 64>(slab_rsrc(krs, live ? (uint32_t)t * ktile : 0u, live), koff,
+                                             kring_lds + (uint32_t)(u & 1) * kPairK + x * (KT_ELEMS * 2) + wave * NKW * 1024);
+      }
+    };
+    auto issue_v = [&](int u) __attribute__((always_inline)) {
+      if (u >= nsteps) return;
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const int t = t_begin + 2 * u + x;
+        const bool live = t * BN < p.N;
+        buffer_load16_to_lds_blocks<NVW, 32>(slab_rsrc(vrs, live ? (uint32_t)t * vtile : 0u, live), voff,
+                                             vring_lds + (uint32_t)(u & 1) * kPairV + x * (VT_ELEMS * 2) + wave * NVW * 1024);
+      }
+    };
+
+    auto run_group = [&](auto G) __attribute__((always_inline)) {
+      constexpr int grp = decltype(G)::value;
+      STile s;
+      u32x4 pk[KC][QT];
+      const uint16_t* klane = smem + grp * KT_ELEMS + lane * 8;
+      const uint16_t* vlane = smem + 4 * KT_ELEMS + grp * VT_ELEMS + lane * 4;
+      // first step of this group whose tile needs the mask (a tile past the range needs it too)
+      int first = n_end / BN;
+      if (p.causal) first = min(first, (wrow0 + 1) / BN);
+      const int mask_from = __builtin_amdgcn_readfirstlane(max(first - t_begin - grp + 1, 0) / 2);
+      auto mma_block = [&](uint32_t tog) __attribute__((always_inline)) {  // S = Q K_j^T, O += P_{j-1} V_{j-1}
+        __builtin_amdgcn_s_setprio(1);
+        qk(s, qf, klane + tog * (2 * KT_ELEMS));
+        pv(acc, pk, vlane + (1 - tog) * (2 * VT_ELEMS), lsum);
+        m_schedule<8>();
+        __builtin_amdgcn_s_setprio(0);
+      };
+      auto softmax_block = [&](int u) __attribute__((always_inline)) {
+        if (u >= nsteps) return;
+        const int n0 = (t_begin + 2 * u + grp) * BN;
+        if (u >= mask_from) mask_tile(s, n0, wrow0, q16, g, n_end, p.causal != 0);
+        float mx[QT];
+        tile_max(s, mx);
+        rescale(mx, acc, ro, l_i, lsum, p.c);
+        exp_pack(s, pk, ro, l_i, p.c);
+      };
+      issue_k(0);
+      wait_vm_lds_barrier<0>();
+      issue_k(1);
+      issue_v(0);
+      if (grp == 0 && wave_has_rows) {
+        qk(s, qf, klane);
+        qk_schedule();
+      }
+      wait_vm_lds_barrier<63>();
+      if (wave_has_rows) {
+        if (grp == 0) {
+          softmax_block(0);
+        } else {
+          qk(s, qf, klane);
+          qk_schedule();
+        }
+      }
+      wait_vm_lds_barrier<0>();
+      int j = 1;
+      if (wave_has_rows) {
+        // unmasked inner steps, as run(): both tiles of the fetched pairs are inside [0, N)
+        const int fast_end = min(min(nsteps - 1, (n_end / BN - t_begin) / 2 - 1), grp == 0 ? mask_from : mask_from + 1);
+        const uint32_t kstep = 2 * ktile, vstep = 2 * vtile;
+        uint32_t tog = 1;  // ring slot of K_j and V_j
+        u32x4 kr = slab_rsrc(krs, (uint32_t)(t_begin + 4) * ktile, true);
+        u32x4 vr = slab_rsrc(vrs, (uint32_t)(t_begin + 2) * vtile, true);
+        const uint32_t kdst = kring_lds + wave * NKW * 1024, vdst = vring_lds + wave * NVW * 1024;
+        for (; j < fast_end; ++j) {
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            buffer_load16_to_lds_blocks<NKW, 64>(slab_rsrc(kr, x * ktile, true), koff,
+                                                 kdst + (1 - tog) * kPairK + x * (KT_ELEMS * 2));
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            buffer_load16_to_lds_blocks<NVW, 32>(slab_rsrc(vr, x * vtile, true), voff,
+                                                 vdst + tog * kPairV + x * (VT_ELEMS * 2));
+          phase_fence();
+          if (grp == 0) mma_block(tog);
+          else softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
+          phase_fence();
+          wait_vm_lds_barrier<63>();
+          phase_fence();
+          if (grp == 0) softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
+          else mma_block(tog);
+          phase_fence();
+          tog = 1 - tog;
+          kr = slab_rsrc(kr, kstep, true);
+          vr = slab_rsrc(vr, vstep, true);
+          wait_vm_lds_barrier<0>();
+          phase_fence();
+        }
+      }
+      for (; j <= nsteps; ++j) {
+        issue_k(j + 1);
+        issue_v(j);
+        if (wave_has_rows) {
+          if (grp == 0) mma_block(j & 1);
+          else softmax_block(j - 1);
+        }
+        wait_vm_lds_barrier<63>();
+        if (wave_has_rows) {
+          if (grp == 0) softmax_block(j);
+          else mma_block(j & 1);
+        }
+        wait_vm_lds_barrier<0>();
+      }
+      // The groups' halves meet: each keeps one half of the d tiles and gets the other group's sums of
+      // them through LDS (the ring is free after the last barrier), with its row offset and row sum.
+      constexpr int HT = DTL / 2, keep0 = grp * HT, give0 = (1 - grp) * HT;
+      float* const ex = reinterpret_cast<float*>(smem);
+      constexpr int kStats = 8 * HT * QT * 256;  // floats before the (m, l) pairs
+      static_assert((kStats + 8 * QT * 128) * 4 <= 4 * (KT_ELEMS + VT_ELEMS) * 2, "exchange fits the ring");
+      float l[QT];
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        l[qt] = kSumMfma ? lsum[qt][0] : xquad_sum(l_i[qt]);
+#pragma unroll
+        for (int i = 0; i < HT; ++i)
+          *reinterpret_cast<floatx4*>(ex + ((wave * HT + i) * QT + qt) * 256 + lane * 4) = acc[give0 + i][qt];
+        ex[kStats + (wave * QT + qt) * 128 + lane] = ro.m[qt];
+        ex[kStats + (wave * QT + qt) * 128 + 64 + lane] = l[qt];
+      }
+      __syncthreads();
+      const int peer = wave ^ 4;
+      constexpr float kLn2 = 0.69314718055994530942f;
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const float m1 = ex[kStats + (peer * QT + qt) * 128 + lane], l1 = ex[kStats + (peer * QT + qt) * 128 + 64 + lane];
+        const float m = fmaxf(ro.m[qt], m1);
+        const float a0 = ro.m[qt] == FA_NEG_INF ? 0.f : fast_exp2((ro.m[qt] - m) * p.c);
+        const float a1 = m1 == FA_NEG_INF ? 0.f : fast_exp2((m1 - m) * p.c);
+        const float lt = l[qt] * a0 + l1 * a1;
+        const float inv = lt > 0.f ? 1.f / lt : 0.f;
+        const float lse_val = lt > 0.f ? (m * p.c + __builtin_amdgcn_logf(lt)) * kLn2 : FA_NEG_INF;
+        floatx4 out[HT];
+#pragma unroll
+        for (int i = 0; i < HT; ++i) {
+          const floatx4 x = *reinterpret_cast<const floatx4*>(ex + ((peer * HT + i) * QT + qt) * 256 + lane * 4);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) out[i][r] = (acc[keep0 + i][qt][r] * a0 + x[r] * a1) * inv;
+        }
+        u32x4 wide[HT / 2];
+        if constexpr (!SPLIT) {  // 64-byte row pieces, as pack_o_wide; cross-lane: before the row test
+#pragma unroll
+          for (int pp = 0; pp < HT / 2; ++pp) {
+            const floatx4 &a = out[2 * pp], &c = out[2 * pp + 1];
+            const auto lo = __builtin_amdgcn_permlane16_swap(T::pack2(a[0], a[1]), T::pack2(c[0], c[1]), false, false);
+            const auto hi2 = __builtin_amdgcn_permlane16_swap(T::pack2(a[2], a[3]), T::pack2(c[2], c[3]), false, false);
+            wide[pp] = (u32x4){lo[0], hi2[0], lo[1], hi2[1]};
+          }
+        }
+        const int i = wrow0 + qt * 16 + q16;
+        if (i < rows) {
+          const int hr = p.pack > 1 ? h + i / p.M : h, mr = p.pack > 1 ? i % p.M : i;
+          if constexpr (SPLIT) {
+            const int64_t wrow = (int64_t)(split * p.B + b) * p.H + hr;
+            float* wo = p.ws_o + (wrow * p.M + mr) * D + keep0 * 16 + 4 * g;
+#pragma unroll
+            for (int d = 0; d < HT; ++d) *reinterpret_cast<floatx4*>(wo + d * 16) = out[d];
+            if (grp == 0 && g == 0) p.ws_lse[wrow * p.M + mr] = lse_val;
+          } else {
+            uint16_t* orow = p.o + (int64_t)b * p.so0 + (int64_t)hr * p.so1 + (int64_t)mr * p.so2 + keep0 * 16;
+#pragma unroll
+            for (int pp = 0; pp < HT / 2; ++pp) *reinterpret_cast<u32x4*>(orow + 32 * pp + wide_col(g)) = wide[pp];
+            if (p.lse != nullptr && grp == 0 && g == 0)
+              p.lse[(int64_t)b * p.sl0 + (int64_t)hr * p.sl1 + (int64_t)mr * p.sl2] = lse_val;
+          }
+        }
+      }
+    };
+    if (wave < 4) run_group(std::integral_constant<int, 0>{});
+    else run_group(std::integral_constant<int, 1>{});
+  }
 };
 
 template <typename Tag, int D, int WAVES, int BN, int PIPE, bool SPLIT>
@@ -1118,7 +1407,9 @@ __global__ __launch_bounds__(WAVES * 64, (Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>:
     FwdParams p) {
   static_assert(kernel_has_sole_arg<FwdParams>(&fa_fwd16_kernel<Tag, D, WAVES, BN, PIPE, SPLIT>),
                 "the epilogues read FwdParams from kernel-argument offset 0: it must stay the only argument");
-  if constexpr (PIPE == 3)
+  if constexpr (PIPE == 4)
+    Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>::run_key_groups(p);
+  else if constexpr (PIPE == 3)
     Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>::run_persistent(p);
   else
     Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>::run(p);
@@ -1136,9 +1427,15 @@ __global__ __launch_bounds__(WAVES * 64, (Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>:
    FA16_SYMBOL(TAG, D, W, BN, PI, SP)}
 #define FA16_PAIR(TAG, DTYPE, D, BN, PI) FA16_ENTRY(TAG, DTYPE, D, 4, BN, PI, 0), FA16_ENTRY(TAG, DTYPE, D, 4, BN, PI, 1)
 #define FA16_PAIR8(TAG, DTYPE, D, BN, PI) FA16_ENTRY(TAG, DTYPE, D, 8, BN, PI, 0), FA16_ENTRY(TAG, DTYPE, D, 8, BN, PI, 1)
+// key groups: 8 waves on 128 rows
+#define FA16_KG_ENTRY(TAG, DTYPE, D, SP)                                                                    \
+  {10, DTYPE, D, 8, 16, 64, SP, (const void*)&fa_fwd16_kernel<TAG, D, 8, 64, 4, (SP != 0)>, \
+   FA16_SYMBOL(TAG, D, 8, 64, 4, SP)}
+#define FA16_KG_PAIR(TAG, DTYPE, D) FA16_KG_ENTRY(TAG, DTYPE, D, 0), FA16_KG_ENTRY(TAG, DTYPE, D, 1)
 #define FA16_ENTRIES(TAG, DTYPE, D)                                                             \
   FA16_PAIR(TAG, DTYPE, D, 64, 0), FA16_PAIR(TAG, DTYPE, D, 32, 0), FA16_PAIR(TAG, DTYPE, D, 64, 1), \
-      FA16_PAIR(TAG, DTYPE, D, 32, 1), FA16_PAIR8(TAG, DTYPE, D, 64, 2), FA16_PAIR8(TAG, DTYPE, D, 64, 3)
+      FA16_PAIR(TAG, DTYPE, D, 32, 1), FA16_PAIR8(TAG, DTYPE, D, 64, 2), FA16_PAIR8(TAG, DTYPE, D, 64, 3), \
+      FA16_KG_PAIR(TAG, DTYPE, D)
 
 static const FaKernelEntry kFwd16Entries[] = {
     FA16_ENTRIES(f16_t, FA_DTYPE_F16, 64),        FA16_ENTRIES(f16_t, FA_DTYPE_F16, 128),

@@ -47,13 +47,15 @@ VARIANT_BY_KERNEL = {
 #   8  ping-pong: 8 waves in two groups of four that alternate MFMA phases and softmax phases
 #      on the same SIMDs (16x16x32 MFMA tiles, 256 query rows per workgroup),
 #   9  the ping-pong kernel in a persistent grid: one workgroup per CU walks a fixed sequence of
-#      query blocks and fetches the next block's Q, K and V during the current block's last steps.
-# The basic variant uses stages 1; optimized and sliced use 2 to 9.
+#      query blocks and fetches the next block's Q, K and V during the current block's last steps,
+#  10  the ping-pong schedule with both groups on the same 128 rows and alternate KV tiles.
+# The basic variant uses stages 1; optimized and sliced use 2 to 10.
 FA_TILE_SPACE = [
     (256, 64, 8, 8),
     (128, 32, 4, 6),
     (128, 64, 4, 7),
     (256, 64, 8, 9),
+    (128, 64, 8, 10),
     (128, 64, 4, 3),
     (256, 64, 8, 3),
     (128, 32, 4, 3),
@@ -80,8 +82,8 @@ FA_TILE_SPACE = [
 ]
 STAGES_BY_VARIANT = {
     hip_lib.FA_VARIANT_BASIC: (1,),
-    hip_lib.FA_VARIANT_OPT: (3, 4, 5, 6, 7, 8, 9, 2),
-    hip_lib.FA_VARIANT_SLICED: (3, 4, 5, 6, 7, 8, 9, 2),
+    hip_lib.FA_VARIANT_OPT: (3, 4, 5, 6, 7, 8, 9, 10, 2),
+    hip_lib.FA_VARIANT_SLICED: (3, 4, 5, 6, 7, 8, 9, 10, 2),
 }
 
 # GEMM tiles in preference order: (block_m, block_n, block_k, waves).
@@ -291,17 +293,54 @@ def _gemm_ranked_tiles(entry: dict) -> list[tuple[tuple[int, ...], int]]:
     return ranked
 
 
+PERSISTENT_TILE = (256, 64, 8, 9)
+KEY_GROUP_TILE = (128, 64, 8, 10)
+# A step of the key-group kernel (both groups' tiles) takes this many steps of the ping-pong kernel: it
+# has the same matrix and softmax work but fetches twice the K/V (D = 128: 2.2 us against 1.6).
+KEY_GROUP_STEP = 1.35
+
+
+def _serial_steps(rows: int, tiles_per_step: int, BH: int, M: int, N: int, causal: bool) -> float:
+    """Steps until the last of BH * ceil(M / rows) blocks ends, one workgroup per CU: the longest block's,
+    or the CUs' share of all blocks' when that is more (equal blocks run in whole rounds)."""
+    blocks = math.ceil(M / rows)
+
+    def steps(i: int) -> int:
+        keys = min(N, (i + 1) * rows) if causal else N
+        return math.ceil(math.ceil(keys / 64) / tiles_per_step)
+
+    if not causal:
+        return math.ceil(BH * blocks / NUM_CUS) * steps(0)
+    return max(steps(blocks - 1), BH * sum(steps(i) for i in range(blocks)) / NUM_CUS)
+
+
+def key_groups_win(BH: int, M: int, N: int, causal: bool) -> bool:
+    """Do 128-row blocks with two key groups end before 256-row ping-pong blocks? True where the latter
+    leave CUs idle: B1 H12 causal N=4096 (192 blocks, the longest 64 steps) 94 -> 70 us, B2 H16 777x1283
+    D64 (128 blocks) 26 -> 19, B1 H28 N=1024 29 -> 22; false at B1 H12 causal N=8192 (204 against 230)."""
+    return KEY_GROUP_STEP * _serial_steps(128, 2, BH, M, N, causal) < _serial_steps(256, 1, BH, M, N, causal)
+
+
 def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M: int, N: int,
                    candidates: list[FaTileChoice]) -> FaTileChoice:
     """Timed-table winner among candidates (the shape's bucket, else its nearest swept bucket of the
-    same variant, dtype, head dim and causality), else the first candidate (preference order)."""
-    entry = _nearest_fa_entry(load_tune_table()["fa"], fa_table_key(variant, dtype, D, causal, B, H, M, N))
+    same variant, dtype, head dim and causality), else the first candidate (preference order). Where
+    that is a ping-pong or key-group tile of another bucket, key_groups_win says which of the two the
+    shape takes (a split-KV launch of few rows fills the chip by splitting: it keeps the tile)."""
+    table, key = load_tune_table()["fa"], fa_table_key(variant, dtype, D, causal, B, H, M, N)
+    entry = _nearest_fa_entry(table, key)
+    by_tile = {(c.block_m, c.block_n, c.waves, c.stages): c for c in reversed(candidates)}
+    best = candidates[0]
     if entry is not None:
         want = tuple(entry["tile"])
-        for c in candidates:
-            if (c.block_m, c.block_n, c.waves, c.stages)[:len(want)] == want:
-                return c
-    return candidates[0]
+        best = next((c for t, c in reversed(by_tile.items()) if t[:len(want)] == want), best)
+    few_rows = variant == hip_lib.FA_VARIANT_SLICED and M < KEY_GROUP_TILE[0]
+    if key not in table and best.stages in (8, 9, 10) and not few_rows:
+        if key_groups_win(B * H, M, N, causal):
+            return by_tile.get(KEY_GROUP_TILE, best)
+        if best.stages == 10:
+            return by_tile.get(PERSISTENT_TILE, best)
+    return best
 
 
 @functools.lru_cache(maxsize=256)

@@ -45,7 +45,7 @@ enum { FA_DTYPE_F16 = 0, FA_DTYPE_BF16 = 1 };
 /* The three reference kernels (flash_atten.py:364-368). */
 enum { FA_VARIANT_BASIC = 0, FA_VARIANT_OPT = 1, FA_VARIANT_SLICED = 2 };
 
-/* One attention tile configuration. block_m = waves * rows_per_wave (rows_per_wave in {32, 64});
+/* One attention tile configuration. block_m = waves * rows_per_wave (rows_per_wave in {32, 64}; 16 for stages 10);
  * block_n = KV rows per LDS tile; splits = KV splits of the sliced variant (1 = no split, no merge
  * pass). stages selects the K/V pipeline of the optimized and sliced variants (basic always runs
  * stages 1):
@@ -67,9 +67,12 @@ enum { FA_VARIANT_BASIC = 0, FA_VARIANT_OPT = 1, FA_VARIANT_SLICED = 2 };
  *      query blocks; the last steps of a block fetch the next block's Q, K and V, so blocks start
  *      without waiting on memory). Launches whose query heads fa_fwd_pack_group would pack, or
  *      whose Q rows (M * q_stride[2] * 2 bytes) reach 2^32, run the stages=8 kernel instead.
- *   The LDS-DMA kernels (3-9) need (N + block_n) * max(k_stride[2], v_stride[2]) * 2 < 2^32
- *   bytes and row strides >= D; when a launch breaks either rule, fa_fwd runs the stages=2 kernel
- *   of the same block_m and waves instead (same block_n where built, else 64). fa_fwd_supported()
+ *   10 key groups (block_m 128, 8 waves, block_n 64, D <= 128): the stages=8 schedule with both groups
+ *      of four waves on the same 128 rows, taking alternate KV tiles; their sums meet in LDS. For
+ *      grids too small to fill the chip with 256-row blocks.
+ *   The LDS-DMA kernels (3-10) need (N + block_n) * max(k_stride[2], v_stride[2]) * 2 < 2^32
+ *   bytes (stages 10: N + 2 * block_n) and row strides >= D; when a launch breaks either rule, fa_fwd runs the stages=2 kernel
+ *   of the same block_m and waves instead (stages 10: 4 waves; same block_n where built, else 64). fa_fwd_supported()
  *   reports such a tile as built only when that fallback is built too. */
 typedef struct {
   int32_t block_m;

@@ -283,6 +283,44 @@ def test_fa_ping_pong_masked_range(gpu, stages, M, N, causal, splits):
     assert max_abs(lse, lse_ref) <= 1e-3
 
 
+KEY_GROUP_CASES = [
+    # B, H, Hkv, M, N, D, dtype, causal, splits: 1 key; one tile of a pair; a pair; odd tile counts with
+    # ragged ends; waves and query tiles without rows; diagonals inside a pair; empty, odd and packed splits
+    (1, 2, 1, 1, 1, 64, F16, False, 1), (1, 2, 2, 33, 64, 128, BF16, False, 1), (2, 3, 3, 128, 128, 128, F16, True, 1),
+    (1, 4, 2, 200, 129, 64, BF16, False, 1), (1, 2, 2, 257, 193, 128, F16, True, 1), (2, 4, 2, 500, 500, 64, F16, True, 1),
+    (1, 2, 1, 300, 1000, 128, BF16, False, 1), (1, 12, 2, 700, 700, 128, BF16, True, 1),
+    (1, 2, 2, 130, 449, 128, F16, False, 3), (1, 2, 1, 640, 640, 64, BF16, True, 4), (1, 8, 2, 2, 900, 128, F16, False, 5),
+]
+
+
+@pytest.mark.parametrize("case", KEY_GROUP_CASES, ids=["x".join(map(str, c[:6])) + f"_c{int(c[7])}_s{c[8]}" for c in KEY_GROUP_CASES])
+def test_fa_key_groups(gpu, case):
+    """stages=10: the two wave groups of a workgroup take alternate KV tiles of the same rows and their
+    sums meet in LDS; O and LSE against the oracle."""
+    B, H, Hkv, M, N, D, dtype, causal, splits = case
+    print(f"[fa_abi] key groups {case}", flush=True)
+    q, k, v = make_qkv(990 + M + N, B, H, Hkv, M, N, D, dtype)
+    variant = SLICED if splits > 1 else OPT
+    o, lse = run_fa(q, k, v, variant=variant, tile=(variant, 128, 64, 8, 10), causal=causal, dtype=dtype, splits=splits)
+    o_ref, lse_ref = oracle.attention(q, k, v, causal=causal)
+    assert max_abs(o, o_ref) <= ATOL[dtype]
+    assert max_abs(lse, lse_ref) <= 1e-3
+
+
+def test_fa_key_groups_fallback_and_stage_numbers(gpu):
+    """A K/V row stride below D runs the 4-wave double-buffered kernel of the same rows; stages=10 on any
+    other tile still means the double-buffered kernel."""
+    q, k, v = (torch.randn(1, 2, s, 128, device="cuda:0", dtype=F16) for s in (200, 300, 300))
+    flat = torch.randn(2 * 301 * 64, device="cuda:0", dtype=F16)
+    view = flat.as_strided((1, 2, 300, 128), (2 * 301 * 64, 301 * 64, 64, 1))
+    outs = []
+    for tile, keys in (((128, 64, 8, 10), view), ((128, 64, 4, 2), view), ((128, 64, 4, 10), k), ((128, 64, 4, 2), k)):
+        o = torch.empty_like(q)
+        hip_lib.fa_fwd(q, keys, keys, o, None, sm_scale=0.1, causal=False, variant=OPT, tile=hip_lib.make_tile(*tile))
+        outs.append(o)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[2], outs[3])
+
+
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
 def test_fa_parity(gpu, case):
     name, B, H, Hkv, M, N, D, dtype, causal, tile_name = case
