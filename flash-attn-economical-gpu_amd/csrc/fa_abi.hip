@@ -45,13 +45,15 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 const fa::FaKernelEntry* find_fwd(int stages, int dtype, int D, int waves, int rows_per_wave, int block_n,
                                   int split) {
-  // stages 1-5: fa_fwd.hip (32x32x16 MFMAs); stages 6-10: fa_fwd16.hip (16x16x32 MFMAs)
-  int n = 0;
-  const fa::FaKernelEntry* e = stages >= 6 ? fa::fa_fwd16_registry(&n) : fa::fa_fwd_registry(&n);
-  for (int i = 0; i < n; ++i)
-    if (e[i].stages == stages && e[i].dtype == dtype && e[i].D == D && e[i].waves == waves &&
-        e[i].rows_per_wave == rows_per_wave && e[i].block_n == block_n && e[i].split == split)
-      return &e[i];
+  // stages 2-5: fa_fwd.hip (32x32x16 MFMAs); stages 6-10: fa_fwd16.hip (16x16x32 MFMAs); 1: either
+  for (int file = stages == 1 || stages >= 6 ? 1 : 0; file >= (stages >= 6 ? 1 : 0); --file) {
+    int n = 0;
+    const fa::FaKernelEntry* e = file == 1 ? fa::fa_fwd16_registry(&n) : fa::fa_fwd_registry(&n);
+    for (int i = 0; i < n; ++i)
+      if (e[i].stages == stages && e[i].dtype == dtype && e[i].D == D && e[i].waves == waves &&
+          e[i].rows_per_wave == rows_per_wave && e[i].block_n == block_n && e[i].split == split)
+        return &e[i];
+  }
   return nullptr;
 }
 
@@ -235,7 +237,7 @@ int fa_fwd_supported(int32_t variant, int32_t dtype, int32_t D, const fa_tile* t
   const fa::FaKernelEntry* e = resolve_fwd(variant, dtype, D, tile, &split, &code);
   if (e == nullptr) return code;
   if (split && find_merge(dtype, D) == nullptr) return fail(FA_ENOTSUP, "no merge kernel for D=%d", D);
-  if (e->stages >= 3 && double_buffered_fallback(e) == nullptr)
+  if (e->pipeline() >= 3 && double_buffered_fallback(e) == nullptr)
     return fail(FA_ENOTSUP, "pipelined tile without a double-buffered fallback for D=%d", D);
   return ok();
 }
@@ -262,7 +264,7 @@ static int launch_fwd(const fa_fwd_args* a, void* ws, int64_t ws_bytes, void* st
   if (!std::isfinite(a->sm_scale) || a->sm_scale <= 0.f)
     return fail(FA_EINVAL, "sm_scale must be positive and finite, got %g", (double)a->sm_scale);
 
-  if (e->stages >= 3 && !pipelined_fits(a, e->stages == 10 ? 2 * e->block_n : e->block_n)) {
+  if (e->pipeline() >= 3 && !pipelined_fits(a, e->pipeline() == 10 ? 2 * e->kv_tile() : e->kv_tile())) {
     // The pipelined kernel addresses one (batch, kv-head) row range [0, N + block_n) of K and V
     // with 32-bit byte offsets and relies on whole rows for its tail check: run the
     // double-buffered kernel of the same rows per workgroup instead (same block_n where it is
@@ -271,14 +273,14 @@ static int launch_fwd(const fa_fwd_args* a, void* ws, int64_t ws_bytes, void* st
     if (fb == nullptr) return fail(FA_ENOTSUP, "no double-buffered fallback for the pipelined attention tile");
     e = fb;
   }
-  const int bm = a->tile.block_m, bn = e->block_n;
+  const int bm = a->tile.block_m, bn = e->kv_tile();
   const int splits = a->tile.splits < 1 ? 1 : a->tile.splits;
   // Decode shapes: when every query row of a GQA group fits in one tile (non-causal), the group's
   // query heads share the tile's rows, so each workgroup reads its kv head's K/V once for all of
   // them instead of once per query head.
   const int group = a->H / a->H_kv;
   const int pack = fa_fwd_pack_group(a->H, a->H_kv, a->M, a->causal, bm, splits);
-  if (e->stages == 9 && (pack > 1 || (int64_t)a->M * a->q_stride[2] * 2 > 0xffffffffLL || a->q_stride[2] < a->D)) {
+  if (e->pipeline() == 9 && (pack > 1 || (int64_t)a->M * a->q_stride[2] * 2 > 0xffffffffLL || a->q_stride[2] < a->D)) {
     // The persistent kernel fetches Q rows of one (batch, head) by LDS-DMA (32-bit offsets, whole
     // rows) and does not pack query heads: the per-workgroup ping-pong kernel runs these launches.
     e = find_fwd(8, e->dtype, e->D, e->waves, e->rows_per_wave, e->block_n, e->split);
@@ -330,7 +332,7 @@ static int launch_fwd(const fa_fwd_args* a, void* ws, int64_t ws_bytes, void* st
   hipStream_t s = static_cast<hipStream_t>(stream);
   void* kargs[] = {&p};
   int64_t grid = total;
-  if (e->stages == 9) {  // persistent: one workgroup per CU (fewer when there are fewer blocks)
+  if (e->pipeline() == 9) {  // persistent: one workgroup per CU (fewer when there are fewer blocks)
     int cus = 0;
     const int code = current_device_cus(&cus);
     if (code != FA_OK) return code;

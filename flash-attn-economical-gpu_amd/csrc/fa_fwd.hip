@@ -1060,14 +1060,13 @@ __global__ __launch_bounds__(256) void fa_merge_kernel(MergeParams p) {
   {ST, DTYPE, D, W, 32 * RT, BN, SP, (const void*)&fa_fwd_kernel<TAG, D, W, RT, BN, ST, (SP != 0)>, \
    FA_SYMBOL(TAG, D, W, RT, BN, ST, SP)}
 
+// (the basic tiles of 64 keys and 32 rows per wave are in fa_fwd16.hip)
 #define FA_ENTRIES_D(TAG, DTYPE, D)                         \
-  FA_ENTRY(TAG, DTYPE, D, 4, 1, 64, 1, 0),                  \
   FA_ENTRY(TAG, DTYPE, D, 4, 1, 64, 2, 0),                  \
   FA_ENTRY(TAG, DTYPE, D, 4, 1, 64, 2, 1)
 
 #define FA_ENTRIES_D_WIDE(TAG, DTYPE, D)                    \
   FA_ENTRY(TAG, DTYPE, D, 4, 2, 64, 1, 0),                  \
-  FA_ENTRY(TAG, DTYPE, D, 8, 1, 64, 1, 0),                  \
   FA_ENTRY(TAG, DTYPE, D, 4, 2, 64, 2, 0),                  \
   FA_ENTRY(TAG, DTYPE, D, 4, 2, 64, 2, 1),                  \
   FA_ENTRY(TAG, DTYPE, D, 8, 1, 64, 2, 0),                  \

@@ -1415,6 +1415,24 @@ __global__ __launch_bounds__(WAVES * 64, (Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>:
     Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>::run(p);
 }
 
+// The basic variant's kernels (stages=1): the bodies above under the basic tiles. 256 rows and 8 waves run
+// the persistent ping-pong, 128 rows and 4 waves the software pipeline, D = 256 the lean pipeline on
+// 32-key tiles. The kernels they replace kept one K/V buffer, filled through registers, with two
+// barriers per tile and 32x32x16 MFMAs: fp16 B4 H32 D128 N=8192 4.29 -> 3.41 ms, causal N=2048 209 -> 143
+// us, bf16 B2 H16 D256 N=2048 180 -> 120 us.
+template <typename Tag, int D, int WAVES, int BN, int STAGES, bool SPLIT>
+__global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 1 : 2) void fa_basic_kernel(FwdParams p) {
+  static_assert(kernel_has_sole_arg<FwdParams>(&fa_basic_kernel<Tag, D, WAVES, BN, STAGES, SPLIT>),
+                "the epilogues read FwdParams from kernel-argument offset 0: it must stay the only argument");
+  static_assert(STAGES == 1 && BN == 64 && !SPLIT, "basic tiles");
+  if constexpr (WAVES == 8)
+    Fwd16<Tag, D, 8, 64, 3, false>::run_persistent(p);
+  else if constexpr (D <= 128)
+    Fwd16<Tag, D, 4, 64, 1, false>::run(p);
+  else
+    Fwd16<Tag, D, 4, 32, 0, false>::run(p);
+}
+
 // Registry (stages=6: PIPE 0, stages=7: PIPE 1, stages=8: PIPE 2 and stages=9: PIPE 3 with 8 waves;
 // 32 query rows per wave).
 #define FA16_SYM_TAG_f16_t "5f16_t"
@@ -1437,7 +1455,15 @@ __global__ __launch_bounds__(WAVES * 64, (Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>:
       FA16_PAIR(TAG, DTYPE, D, 32, 1), FA16_PAIR8(TAG, DTYPE, D, 64, 2), FA16_PAIR8(TAG, DTYPE, D, 64, 3), \
       FA16_KG_PAIR(TAG, DTYPE, D)
 
+#define FA16_BASIC(TAG, DTYPE, D, W, BODY, BODY_BN)                                                    \
+  {1, DTYPE, D, W, 32, 64, 0, (const void*)&fa_basic_kernel<TAG, D, W, 64, 1, false>,                 \
+   "_ZN2fa15fa_basic_kernelINS_" FA16_SYM_TAG_##TAG "ELi" #D "ELi" #W "ELi64ELi1ELb0EEEvNS_9FwdParamsE", BODY, BODY_BN}
+#define FA16_BASICS(TAG, DTYPE)                                                                 \
+  FA16_BASIC(TAG, DTYPE, 64, 8, 9, 64), FA16_BASIC(TAG, DTYPE, 64, 4, 7, 64), FA16_BASIC(TAG, DTYPE, 128, 8, 9, 64), \
+      FA16_BASIC(TAG, DTYPE, 128, 4, 7, 64), FA16_BASIC(TAG, DTYPE, 256, 4, 6, 32)
+
 static const FaKernelEntry kFwd16Entries[] = {
+    FA16_BASICS(f16_t, FA_DTYPE_F16),             FA16_BASICS(bf16_t, FA_DTYPE_BF16),
     FA16_ENTRIES(f16_t, FA_DTYPE_F16, 64),        FA16_ENTRIES(f16_t, FA_DTYPE_F16, 128),
     FA16_ENTRIES(bf16_t, FA_DTYPE_BF16, 64),      FA16_ENTRIES(bf16_t, FA_DTYPE_BF16, 128),
     // D = 256: one tile per step only (the pipelined kernel's two score tiles do not fit beside O

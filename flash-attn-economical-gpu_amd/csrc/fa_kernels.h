@@ -49,9 +49,9 @@ typedef void (*FwdKernelFn)(FwdParams);
 typedef void (*MergeKernelFn)(MergeParams);
 
 struct FaKernelEntry {
-  int32_t stages;  // 1 = single-buffered K/V LDS (basic), 2 = double-buffered (optimized),
-                   // 3-5 = LDS-DMA pipelines (32x32x16 MFMAs), 6-9 = 16x16x32 MFMA kernels: 6 lean,
-                   // 7 software-pipelined, 8 ping-pong, 9 persistent ping-pong (fa_fwd16.hip)
+  int32_t stages;  // 1 = basic, 2 = double-buffered K/V LDS (optimized), 3-5 = LDS-DMA pipelines
+                   // (32x32x16 MFMAs), 6-10 = 16x16x32 MFMA kernels: 6 lean, 7 software-pipelined,
+                   // 8 ping-pong, 9 persistent ping-pong, 10 key groups (fa_fwd16.hip)
   int32_t dtype;   // FA_DTYPE_*
   int32_t D;
   int32_t waves;
@@ -60,6 +60,12 @@ struct FaKernelEntry {
   int32_t split;   // writes fp32 partials for the LSE merge
   const void* fn;
   const char* symbol;  // mangled kernel name (the key of the build's resource table)
+  // The basic kernels of fa_fwd16.hip run the body of another stages number: its launch rules apply
+  // (addressing limits, grid), and its KV tile may be smaller than the block_n the tile names.
+  int32_t body_stages = 0;
+  int32_t body_block_n = 0;
+  int32_t pipeline() const { return body_stages ? body_stages : stages; }
+  int32_t kv_tile() const { return body_block_n ? body_block_n : block_n; }
 };
 
 struct FaMergeEntry {

@@ -34,7 +34,8 @@ VARIANT_BY_KERNEL = {
 # Attention tiles in preference order (used when the tuning table has no entry for a shape's variant,
 # dtype, head dim and causality; the first ones are the fastest measured at large sizes):
 # (block_m, block_n, waves, stages). stages selects the kernel pipeline:
-#   1  one K/V buffer, two barriers per KV tile (the basic variant),
+#   1  the basic variant: the bodies of stages 9, 7 and 6 (64 keys, 32 rows per wave), else one K/V
+#      buffer with two barriers per KV tile,
 #   2  double-buffered K/V, one barrier per tile,
 #   3  software-pipelined (QK of tile u+1 overlapped with the softmax of tile u inside each wave,
 #      K/V brought into an LDS ring by LDS-DMA loads),

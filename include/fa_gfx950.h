@@ -49,7 +49,9 @@ enum { FA_VARIANT_BASIC = 0, FA_VARIANT_OPT = 1, FA_VARIANT_SLICED = 2 };
  * block_n = KV rows per LDS tile; splits = KV splits of the sliced variant (1 = no split, no merge
  * pass). stages selects the K/V pipeline of the optimized and sliced variants (basic always runs
  * stages 1):
- *   1  one K/V LDS buffer, staged through registers;
+ *   1  the basic kernels: with 64-key tiles and 32 rows per wave the body of stages 9 (8 waves), 7 (4
+ *      waves) or 6 (D = 256), each with its rules below; the other tiles keep one K/V LDS buffer,
+ *      staged through registers;
  *   2  double-buffered K/V LDS tiles, staged through registers;
  *   3  software-pipelined kernel: K/V reach a ring of LDS tiles by LDS-DMA, and the QK^T MFMAs of
  *      tile u+1 run beside the softmax of tile u;

@@ -283,6 +283,30 @@ def test_fa_ping_pong_masked_range(gpu, stages, M, N, causal, splits):
     assert max_abs(lse, lse_ref) <= 1e-3
 
 
+@pytest.mark.parametrize("D,tile,body", [(64, (256, 64, 8), (256, 64, 8, 9)), (128, (256, 64, 8), (256, 64, 8, 9)),
+                                         (128, (128, 64, 4), (128, 64, 4, 7)), (256, (128, 64, 4), (128, 32, 4, 6))])
+@pytest.mark.parametrize("M,N,causal", [(1, 1, False), (200, 33, False), (130, 95, True), (300, 700, False), (1000, 1000, True)])
+def test_fa_basic_bodies(gpu, D, tile, body, M, N, causal):
+    """The basic tiles of 64 keys run the body of another stages number (at D = 256 on 32-key tiles):
+    bit for bit that kernel's output, also where K/V rows shorter than D send both to the
+    double-buffered kernel."""
+    print(f"[fa_abi] basic body D={D} {tile} M={M} N={N} causal={causal}", flush=True)
+    g = torch.Generator(device="cuda:0").manual_seed(M + N)
+    q = torch.randn(2, 3, M, D, device="cuda:0", generator=g).to(BF16)
+    kv = torch.randn(2, 3, N + 1, D, device="cuda:0", generator=g).to(BF16)
+    short = torch.randn(6 * (N + 1) * (D // 2) + D, device="cuda:0", generator=g).to(BF16).as_strided(
+        (2, 3, N, D), (3 * (N + 1) * (D // 2), (N + 1) * (D // 2), D // 2, 1))
+    for keys in (kv[:, :, :N], short):
+        outs = []
+        for variant, t in ((BASIC, (*tile, 1)), (OPT, body)):
+            o = torch.full_like(q, float("nan"))
+            lse = torch.full((2, 3, M), float("nan"), device="cuda:0")
+            hip_lib.fa_fwd(q, keys, keys, o, lse, sm_scale=0.09, causal=causal, variant=variant, tile=hip_lib.make_tile(*t))
+            outs.append((o, lse))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+        assert bool(torch.isfinite(outs[0][0]).all())
+
+
 KEY_GROUP_CASES = [
     # B, H, Hkv, M, N, D, dtype, causal, splits: 1 key; one tile of a pair; a pair; odd tile counts with
     # ragged ends; waves and query tiles without rows; diagonals inside a pair; empty, odd and packed splits
