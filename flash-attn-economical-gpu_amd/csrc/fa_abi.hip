@@ -387,6 +387,10 @@ int fa_fwd_noalloc(const fa_fwd_args* a, void* stream) {
   return launch_fwd(a, ptr, kScratchBytes, stream);
 }
 
+int64_t gemm_f16_workspace_bytes(int32_t M, int32_t N, int32_t ksplits) {
+  return ksplits <= 1 || M <= 0 || N <= 0 ? 0 : (int64_t)ksplits * M * N * 4;
+}
+
 int gemm_f16_supported(const gemm_tile* tile) {
   if (tile == nullptr) return fail(FA_EINVAL, "null gemm tile");
   if (find_gemm(tile) == nullptr)
@@ -401,7 +405,8 @@ int gemm_f16_supported(const gemm_tile* tile) {
 // now and then. Against restaging B into rows of a 16-byte pitch (a fill and a copy before the product),
 // time per call: 1000x1004x1000 59 -> 48 us, 4000x4004x4000 148 -> 119, 8000x8004x8000 879 -> 811.
 static int launch_gemm(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K, int64_t lda,
-                       int64_t ldb, int64_t ldc, const gemm_tile* tile, void* stream, int ldb_step) {
+                       int64_t ldb, int64_t ldc, const gemm_tile* tile, void* stream, int ldb_step, int32_t ksplits = 1,
+                       void* ws = nullptr, int64_t ws_bytes = 0) {
   if (tile == nullptr) return fail(FA_EINVAL, "null gemm tile");
   const fa::GemmKernelEntry* e = find_gemm(tile);
   if (e == nullptr)
@@ -427,6 +432,7 @@ static int launch_gemm(const void* a, const void* b, void* c, int32_t M, int32_t
     return fail(FA_ENOTSUP, "GEMM operand spans beyond 2 GiB per tile (lda=%lld ldb=%lld K=%d)", (long long)lda,
                 (long long)ldb, K);
   fa::GemmParams p;
+  std::memset(&p, 0, sizeof(p));
   p.a = static_cast<const uint16_t*>(a);
   p.b = static_cast<const uint16_t*>(b);
   p.c = static_cast<uint16_t*>(c);
@@ -437,6 +443,25 @@ static int launch_gemm(const void* a, const void* b, void* c, int32_t M, int32_t
   p.tiles_n = (N + e->block_n - 1) / e->block_n;
   const int64_t total = (int64_t)p.tiles_m * p.tiles_n;
   if (total > 0x7fffffffLL) return fail(FA_EINVAL, "grid too large");
+  if (ksplits > 1) {
+    if (e->fn_part == nullptr) return fail(FA_ENOTSUP, "no split-K kernel for this GEMM tile");
+    const int64_t need = gemm_f16_workspace_bytes(M, N, ksplits);
+    if (ws == nullptr || ws_bytes < need)
+      return fail(FA_EWORKSPACE, "split-K workspace of %lld bytes needed, got %lld", (long long)need, (long long)ws_bytes);
+    if (!aligned16(ws)) return fail(FA_EINVAL, "workspace must be 16-byte aligned");
+    const int all = (K + e->block_k - 1) / e->block_k;
+    p.ws = static_cast<float*>(ws);
+    p.slabs_per_split = (all + ksplits - 1) / ksplits;
+    p.ksplits = (all + p.slabs_per_split - 1) / p.slabs_per_split;  // no empty split
+    const int64_t wgs = total * p.ksplits, chunks = ((int64_t)M * N / 4 + 255) / 256;
+    if (wgs > 0x7fffffffLL || chunks > 0x7fffffffLL) return fail(FA_EINVAL, "grid too large");
+    void* pargs[] = {&p};
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    hipError_t perr = hipLaunchKernel(e->fn_part, dim3((unsigned)wgs), dim3((unsigned)e->waves * 64), pargs, 0, s);
+    if (perr == hipSuccess) perr = hipLaunchKernel(fa::gemm_reduce_fn(), dim3((unsigned)chunks), dim3(256), pargs, 0, s);
+    if (perr != hipSuccess) return fail(FA_EHIP, "split-K gemm launch failed: %s", hipGetErrorString(perr));
+    return ok();
+  }
   p.region_m = gemm_region_rows(p.tiles_m, p.tiles_n, e->block_m, e->block_n);
   // Short K loops run the tile's shallow-ring kernel where one is built (more workgroups per CU),
   // or its persistent kernel (one workgroup per CU overlapping each tile's C write with the next
@@ -470,6 +495,13 @@ int gemm_f16(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_
 int gemm_f16_ldb4(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K, int64_t lda, int64_t ldb,
                   int64_t ldc, const gemm_tile* tile, void* stream) {
   return launch_gemm(a, b, c, M, N, K, lda, ldb, ldc, tile, stream, 4);
+}
+
+int gemm_f16_splitk(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K, int64_t lda, int64_t ldb,
+                    int64_t ldc, const gemm_tile* tile, int32_t ksplits, void* workspace, int64_t workspace_bytes,
+                    void* stream) {
+  if (ksplits < 1) return fail(FA_EINVAL, "ksplits=%d must be >= 1", ksplits);
+  return launch_gemm(a, b, c, M, N, K, lda, ldb, ldc, tile, stream, 4, ksplits, workspace, workspace_bytes);
 }
 
 // The built kernel an (op, variant, dtype, D, tile) or GEMM tile resolves to: its function, mangled

@@ -88,6 +88,10 @@ struct GemmParams {
   int32_t tiles_m, tiles_n;
   int32_t region_m;  // 0: flat grouped order; else XCD regions in region_m rows x (8 / region_m) columns
   int32_t grid;      // workgroups launched (the persistent kernel walks tiles with this stride)
+  // split K over the grid (gemm_f16_part_kernel, gemm_f16_reduce_kernel)
+  float* ws;                // fp32 partial products [ksplits][M][N]
+  int32_t ksplits;
+  int32_t slabs_per_split;  // K slabs (of block_k) per split
 };
 
 struct GemmKernelEntry {
@@ -96,6 +100,7 @@ struct GemmKernelEntry {
   const void* fn_shallow;  // shallow ring for short K (nullptr when it would be the same)
   const char* symbol;      // mangled name of `fn`
   const void* fn_persist;  // persistent short-K kernel (nullptr when not built for the tile)
+  const void* fn_part = nullptr;  // split-K kernel (nullptr when not built for the tile)
 };
 
 // K slabs up to which a tile's shallow-ring kernel is launched (more workgroups per CU beat a
@@ -110,6 +115,7 @@ constexpr int kGemmPersistMaxSlabs = 16;
 constexpr int kGemmPersistStoreWaves = 4;
 
 const GemmKernelEntry* gemm_registry(int* count);
+const void* gemm_reduce_fn();
 
 // Resources of one kernel as the compiler reported them (-Rpass-analysis=kernel-resource-usage).
 // The table is generated by build_lib.py after the kernels are compiled and linked into the

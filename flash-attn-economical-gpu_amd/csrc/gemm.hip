@@ -323,7 +323,12 @@ struct GemmKernel {
     }
   }
 
+  // PART: the grid splits K too (gemm_f16_part_kernel): workgroup w multiplies split w % ksplits of
+  // tile w / ksplits and leaves fp32 sums in the workspace. With 2, 4 or 8 splits a split's slices of A
+  // and B are read by one share of the XCDs only.
+  template <bool PART = false>
   __device__ static void run(const GemmParams& p) {
+    static_assert(!PART || (KSG > 1 && MI == 32), "split-K kernels: the K-group tiles");
     __shared__ __attribute__((aligned(16))) char smem[SMEM_BYTES];
     const int tid = (int)__builtin_amdgcn_workitem_id_x();
     const int lane = tid & 63;
@@ -333,8 +338,14 @@ struct GemmKernel {
     const int col = lane & 31, hh = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
 
-    int pid_m, pid_n;
-    if (p.region_m > 0) {
+    int pid_m, pid_n, part = 0;
+    if constexpr (PART) {
+      const int wg = (int)__builtin_amdgcn_workgroup_id_x();
+      part = __builtin_amdgcn_readfirstlane(wg % p.ksplits);
+      const int tile = wg / p.ksplits;
+      pid_m = __builtin_amdgcn_readfirstlane(tile % p.tiles_m);
+      pid_n = __builtin_amdgcn_readfirstlane(tile / p.tiles_m);
+    } else if (p.region_m > 0) {
       // XCD x (workgroups are dispatched round-robin: blockIdx % 8) owns one rectangle of tiles,
       // region (x / rn, x % rn) of a region_m x rn split, and walks it in GROUP_M-grouped order:
       // each XCD's L2 then sees tiles_m / region_m A panels and tiles_n / rn B panels instead of
@@ -477,15 +488,17 @@ struct GemmKernel {
       // K group kg multiplies slabs kbase .. kbase + per - 1 (its step ks is slab kbase + ks) in its
       // own ring; all groups take the same steps and barriers, a group's steps past its run or past
       // K multiplying zeros.
-      const int per = KSG == 1 ? ksteps : (ksteps + KSG - 1) / KSG;
-      const int kbase = kg * per;
+      const int kfirst = PART ? part * p.slabs_per_split : 0;
+      const int kend = PART ? min(ksteps, kfirst + p.slabs_per_split) : ksteps;
+      const int per = KSG == 1 ? ksteps : (kend - kfirst + KSG - 1) / KSG;
+      const int kbase = kfirst + kg * per;
       const uint32_t ring_lds = smem_lds + (uint32_t)(kg * RING * SLAB_BYTES);
       const char* const ring = smem + kg * RING * SLAB_BYTES;
       auto dma_slab = [&](int ks, auto jc) __attribute__((always_inline)) {
         constexpr int j = decltype(jc)::value;
         const uint32_t slot = ring_lds + (uint32_t)(ks % RING) * SLAB_BYTES;
         const int gk = kbase + ks;
-        const bool live = (ks < per) & (gk < ksteps);
+        const bool live = (ks < per) & (gk < kend);
         // 16x16 tiles: the slab's offset moves the buffer resource (base + offset, range - offset,
         // range 0 past the last slab), so each lane's offset is the same on every step and the
         // DMA takes no vector op; a lane reads zeros exactly where it did with the offset added to
@@ -592,6 +605,28 @@ struct GemmKernel {
           });
         }
       }
+    }
+
+    if constexpr (PART) {
+      // fp32 sums of this split: a lane's 4 consecutive columns per store (N % 4 == 0)
+      if (kg == 0) {
+        float* const wsp = p.ws + (int64_t)part * p.M * p.N;
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm) {
+          const int m = m0 + (wm * TM + tm) * MI + col;
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+#pragma unroll
+            for (int gq = 0; gq < 4; ++gq) {
+              const int n = n0 + (wn * TN + tn) * 32 + 8 * gq + 4 * hh;
+              if (m < p.M && n < p.N)
+                *reinterpret_cast<floatx4*>(wsp + (int64_t)m * p.N + n) =
+                    (floatx4){acc_at(acc, tn, tm, 4 * gq), acc_at(acc, tn, tm, 4 * gq + 1), acc_at(acc, tn, tm, 4 * gq + 2),
+                              acc_at(acc, tn, tm, 4 * gq + 3)};
+            }
+        }
+      }
+      return;
     }
 
     // C goes out through LDS (the ring is free after the last step's barrier): each lane holds 4
@@ -903,6 +938,41 @@ __global__ __launch_bounds__(WM * WN * KSG * 64) void gemm_f16_ksplit_kernel(Gem
   GemmKernel<BM, BN, BK, WM, WN, false, MI, 1, KSG>::run(p);
 }
 
+// A split of K over the grid as well: for products of few tiles and a long K, whose serial slab loop is
+// the time (64x64 tiles: 0.22 us per step of two 32-deep slabs).
+template <int BM, int BN, int BK, int WM, int WN, int MI, int KSG>
+__global__ __launch_bounds__(WM * WN * KSG * 64) void gemm_f16_part_kernel(GemmParams p) {
+  GemmKernel<BM, BN, BK, WM, WN, false, MI, 1, KSG>::template run<true>(p);
+}
+
+// C = the sum of the splits' fp32 partial products, in split order, rounded once. Four columns per thread;
+// four splits' loads in flight. Bound by launch latency and the partials' traffic (they sit in L2 / MALL).
+__global__ __launch_bounds__(256) void gemm_f16_reduce_kernel(GemmParams p) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  const int64_t mn = (int64_t)p.M * p.N;
+  if (i >= mn) return;
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+  const float* src = p.ws + i;
+  int s = 0;
+  for (; s + 4 <= p.ksplits; s += 4) {
+    floatx4 x[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const floatx4*>(src + (s + u) * mn);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[e] += x[u][e];
+  }
+  for (; s < p.ksplits; ++s) {
+    const floatx4 x = *reinterpret_cast<const floatx4*>(src + s * mn);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum[e] += x[e];
+  }
+  const int64_t m = i / p.N, n = i % p.N;
+  *reinterpret_cast<u32x2*>(p.c + m * p.ldc + n) =
+      (u32x2){DT<f16_t>::pack2(sum[0], sum[1]), DT<f16_t>::pack2(sum[2], sum[3])};
+}
+
 // The shallow-ring kernel of a tile, or nullptr when its ring would be as deep as the default one.
 template <int BM, int BN, int BK, int WM, int WN, int MI, int SCHED>
 const void* gemm_shallow_fn() {
@@ -929,6 +999,11 @@ const void* gemm_shallow_fn() {
   {BM, BN, BK, WM * WN * KSG, (const void*)&gemm_f16_ksplit_kernel<BM, BN, BK, WM, WN, MI, KSG>, nullptr, \
    "_ZN2fa22gemm_f16_ksplit_kernelILi" #BM "ELi" #BN "ELi" #BK "ELi" #WM "ELi" #WN "ELi" #MI "ELi" #KSG \
    "EEEvNS_10GemmParamsE", nullptr}
+// The same with its split-K kernel.
+#define GEMM_ENTRY_KSPLIT_PART(BM, BN, BK, WM, WN, MI, KSG)                                               \
+  {BM, BN, BK, WM * WN * KSG, (const void*)&gemm_f16_ksplit_kernel<BM, BN, BK, WM, WN, MI, KSG>, nullptr, \
+   "_ZN2fa22gemm_f16_ksplit_kernelILi" #BM "ELi" #BN "ELi" #BK "ELi" #WM "ELi" #WN "ELi" #MI "ELi" #KSG \
+   "EEEvNS_10GemmParamsE", nullptr, (const void*)&gemm_f16_part_kernel<BM, BN, BK, WM, WN, MI, KSG>}
 
 // One kernel per tile: the MFMA shape and schedule measured fastest for it on MI355X (16x16x32
 // MFMAs draw less power per flop, which raises the clock of the 8-wave tiles; the pipelined
@@ -945,10 +1020,12 @@ static const GemmKernelEntry kGemmEntries[] = {
     GEMM_ENTRY(128, 64, 32, 2, 2, 32, 0),
     GEMM_ENTRY(64, 256, 32, 2, 2, 16, 1),
     GEMM_ENTRY_KSPLIT(128, 128, 32, 2, 2, 32, 2),
-    GEMM_ENTRY_KSPLIT(128, 64, 32, 2, 2, 32, 2),
+    GEMM_ENTRY_KSPLIT_PART(128, 64, 32, 2, 2, 32, 2),
     GEMM_ENTRY_KSPLIT(128, 64, 32, 2, 2, 32, 4),
-    GEMM_ENTRY_KSPLIT(64, 64, 32, 2, 2, 32, 2),
+    GEMM_ENTRY_KSPLIT_PART(64, 64, 32, 2, 2, 32, 2),
 };
+
+const void* gemm_reduce_fn() { return (const void*)&gemm_f16_reduce_kernel; }
 
 const GemmKernelEntry* gemm_registry(int* count) {
   *count = (int)(sizeof(kGemmEntries) / sizeof(kGemmEntries[0]));

@@ -107,6 +107,37 @@ GEMM_TILE_SPACE = [
 ]
 GEMM_DEFAULT_GROUP_M = 8
 
+# Time model of a GEMM tile, (c, lat, thr, r) in us: c + steps * max(lat * ceil(tiles / (256 r)),
+# thr * tiles / 256), with steps the K slabs one K group multiplies, lat a step alone on a CU, thr a
+# step's share of a full chip and r the workgroups a CU holds. Fitted to timings of every tile at 240
+# sizes spread over M, N, K = 64 .. 8192 (mean error 5-15%). The fastest tile by the model is within
+# 3% of the fastest timed one on average; the nearest swept bucket's was 23% slower, at worst 3.9x.
+GEMM_COST = {
+    (256, 256, 64, 8): (5.47, 1.017, 2.531, 1),
+    (256, 256, 64, 4): (7.19, 1.124, 2.720, 4),
+    (256, 256, 32, 8): (6.05, 0.545, 1.181, 4),
+    (256, 256, 32, 4): (7.12, 0.528, 1.185, 3),
+    (256, 128, 64, 8): (4.02, 0.608, 1.708, 2),
+    (128, 256, 64, 8): (3.87, 0.605, 1.599, 3),
+    (128, 128, 64, 4): (4.18, 0.448, 0.913, 2),
+    (128, 128, 32, 4): (3.87, 0.213, 0.432, 1),
+    (128, 64, 32, 4): (3.14, 0.221, 0.266, 1),
+    (64, 256, 32, 4): (3.81, 0.240, 0.391, 1),
+    (128, 128, 32, 8): (4.52, 0.342, 1.062, 2),
+    (128, 64, 32, 8): (3.61, 0.272, 0.648, 3),
+    (128, 64, 32, 16): (4.98, 0.440, 1.360, 4),
+    (64, 64, 32, 8): (3.29, 0.221, 0.362, 1),
+}
+GEMM_GROUPS = {(128, 128, 32, 8): 2, (128, 64, 32, 8): 2, (128, 64, 32, 16): 4, (64, 64, 32, 8): 2}  # K groups
+# Another choice than the timed one is taken when the model puts it this much ahead (its error is smaller).
+GEMM_MODEL_MARGIN = 1.15
+# K split over the grid (hip_lib.gemm_f16 ksplits): the tiles it is built for, and its second launch's time
+# (us) and partial-sum traffic (bytes per us). 74x608x6216 29.9 -> 9.2 us in 8 splits, 64x4096x4096 20.5 ->
+# 12.1 in 4; 1000x1004x1000 (256 tiles) 8.6 -> 14 in 2, which the model refuses.
+GEMM_SPLIT_TILES = ((64, 64, 32, 8), (128, 64, 32, 8))
+GEMM_SPLITS = (2, 3, 4, 6, 8, 12, 16)
+GEMM_SPLIT_US, GEMM_SPLIT_BYTES_PER_US = 2.8, 4e6
+
 # The sliced variant splits KV until every CU holds as many workgroups as the kernel can keep
 # resident (RESIDENT_DEFAULT when its resources are unknown); splitting further only adds merge
 # traffic.
@@ -156,8 +187,13 @@ def fa_candidates(variant: int, dtype, D: int) -> list[FaTileChoice]:
     return out
 
 
+@functools.lru_cache(maxsize=1)
+def _built_gemm_tiles() -> tuple[tuple[int, int, int, int], ...]:
+    return tuple(t for t in GEMM_TILE_SPACE if hip_lib.gemm_supported(hip_lib.GemmTile(t[0], t[1], t[2], t[3], 1)))
+
+
 def gemm_candidates() -> list[tuple[int, int, int, int]]:
-    return [t for t in GEMM_TILE_SPACE if hip_lib.gemm_supported(hip_lib.GemmTile(t[0], t[1], t[2], t[3], 1))]
+    return list(_built_gemm_tiles())
 
 
 # ---- hint resolution ----------------------------------------------------------------------------
@@ -393,6 +429,53 @@ def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_
     return splits_for(max(1, math.ceil(M / block_m) * B * H))
 
 
+def gemm_cost(tile: tuple[int, int, int, int], M: int, N: int, K: int, ksplits: int = 1) -> float:
+    """Modelled time (us) of a product with a tile, its K split over ksplits workgroups per tile."""
+    c, lat, thr, resident = GEMM_COST[tile]
+    tiles = math.ceil(M / tile[0]) * math.ceil(N / tile[1])
+    slabs = math.ceil(K / tile[2])
+    per = math.ceil(slabs / ksplits)
+    parts = math.ceil(slabs / per)
+    steps = math.ceil(per / GEMM_GROUPS.get(tile, 1))
+    us = c + steps * max(lat * math.ceil(tiles * parts / (NUM_CUS * resident)), thr * tiles * parts / NUM_CUS)
+    if ksplits > 1:
+        us += GEMM_SPLIT_US + parts * M * N * 8 / GEMM_SPLIT_BYTES_PER_US
+    return us
+
+
+def _swept_size(M: int, N: int, K: int) -> bool:
+    """The sizes are within a quarter of a swept bucket's own (its upper corner): its timing holds."""
+    return gemm_table_key(M, N, K) in load_tune_table()["gemm"] and all(4 * x > 3 * _bucket(x) for x in (M, N, K))
+
+
+def _runs_persistent(tile: tuple[int, int, int, int], M: int, N: int, K: int) -> bool:
+    """The launch takes the persistent short-K kernel of the 256x128x64 tile, which the model does not know."""
+    return (tile == (256, 128, 64, 8) and M % 256 == 0 and N % 128 == 0 and K % 64 == 0 and 256 <= K <= 1024
+            and (M // 256) * (N // 128) % 8 == 0)
+
+
+def _by_model(choice: tuple[int, int, int, int, int], entry: dict, candidates, M: int, N: int, K: int):
+    """The timed choice, or the timed candidate of the entry that the model puts clearly ahead of it."""
+    if choice[:4] not in GEMM_COST or _swept_size(M, N, K) or _runs_persistent(choice[:4], M, N, K):
+        return choice
+    timed = {t for t, _ in _gemm_ranked_tiles(entry)}
+    best = min((t for t in candidates if t in GEMM_COST and t in timed), key=lambda t: gemm_cost(t, M, N, K),
+               default=choice[:4])
+    if gemm_cost(best, M, N, K) * GEMM_MODEL_MARGIN < gemm_cost(choice[:4], M, N, K):
+        return (*best, GEMM_DEFAULT_GROUP_M)
+    return choice
+
+
+def choose_gemm_splits(M: int, N: int, K: int, tile: tuple[int, int, int, int]) -> tuple[tuple[int, int, int, int], int]:
+    """(tile, ksplits): the given tile unsplit, or a split-K tile the model puts clearly ahead of it."""
+    if tile not in GEMM_COST or _runs_persistent(tile, M, N, K):
+        return tile, 1
+    best = min((gemm_cost(t, M, N, K, s), t, s) for t in GEMM_SPLIT_TILES for s in GEMM_SPLITS)
+    if best[0] * GEMM_MODEL_MARGIN < gemm_cost(tile, M, N, K):
+        return best[1], best[2]
+    return tile, 1
+
+
 def choose_gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None = None) -> tuple[int, int, int, int, int]:
     """(block_m, block_n, block_k, waves, group_m) for a GEMM; ValueError when no built tile divides.
 
@@ -419,12 +502,13 @@ def choose_gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None =
             hinted = [t for t in cands if t[:3] == hint[:3]]
         cands = hinted or cands
     # the bucket's (or nearest swept bucket's) winner when it divides, else its fastest timed tile
-    # that does; the preference order only without a table
+    # that does, unless the time model puts another clearly ahead; the preference order only without a
+    # table
     entry = _nearest_gemm_entry(load_tune_table()["gemm"], gemm_table_key(M, N, K))
     if entry is not None:
         for tile, group_m in _gemm_ranked_tiles(entry):
             if tile in cands:
-                return (*tile, group_m)
+                return _by_model((*tile, group_m), entry, cands, M, N, K)
     t = cands[0]
     return (*t, _gemm_group_m(M, N, K, t))
 
@@ -433,19 +517,20 @@ def choose_gemm_tile_any(M: int, N: int, K: int) -> tuple[int, int, int, int, in
     """(block_m, block_n, block_k, waves, group_m) for any shape the kernel accepts (K % 8 == 0,
     N % 4 == 0; partial tiles in M, N and K are masked in the kernel): the divisible choice when
     there is one, else the tuned tile of the shape's bucket, else the first built tile no larger
-    than the problem (rounded up to 64)."""
+    than the problem (rounded up to 64); the time model's choice where that is clearly ahead."""
     if K % 8 != 0 or N % 4 != 0:
         raise ValueError(f"gfx950 GEMM needs K % 8 == 0 and N % 4 == 0 (got M={M} N={N} K={K})")
-    try:
-        return choose_gemm_tile(M, N, K)
-    except ValueError:
-        pass
     cands = gemm_candidates()
     entry = _nearest_gemm_entry(load_tune_table()["gemm"], gemm_table_key(M, N, K))
+    try:
+        choice = choose_gemm_tile(M, N, K)
+        return _by_model(choice, entry, cands, M, N, K) if entry is not None else choice
+    except ValueError:
+        pass
     if entry is not None:
         for tile, group_m in _gemm_ranked_tiles(entry):
             if tile in cands:
-                return (*tile, group_m)
+                return _by_model((*tile, group_m), entry, cands, M, N, K)
     fit = [t for t in cands if t[0] <= -(-M // 64) * 64 and t[1] <= -(-N // 64) * 64]
     t = (fit or [min(cands, key=lambda t: t[0] * t[1])])[0]
     return (*t, GEMM_DEFAULT_GROUP_M)

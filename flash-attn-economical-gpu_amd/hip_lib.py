@@ -131,6 +131,16 @@ SIGNATURES = {
             ctypes.POINTER(GemmTile), ctypes.c_void_p,
         ],
     ),
+    "gemm_f16_splitk": (
+        ctypes.c_int,
+        [
+            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
+            ctypes.c_int32, ctypes.c_int32, ctypes.c_int32,
+            ctypes.c_int64, ctypes.c_int64, ctypes.c_int64,
+            ctypes.POINTER(GemmTile), ctypes.c_int32, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+        ],
+    ),
+    "gemm_f16_workspace_bytes": (ctypes.c_int64, [ctypes.c_int32] * 3),
     "gemm_f16_supported": (ctypes.c_int, [ctypes.POINTER(GemmTile)]),
     "fa_kernel_resources": (
         ctypes.c_int,
@@ -356,9 +366,11 @@ def fa_fwd_noalloc(
     check(lib.fa_fwd_noalloc(ctypes.byref(args), _stream_ptr(q.device)), "fa_fwd_noalloc")
 
 
-def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile, *, ldb4: bool = False) -> None:
+def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile, *, ldb4: bool = False,
+             ksplits: int = 1) -> None:
     """C = A @ B (fp16, fp32 accumulation) written into c on the current stream. ldb4: B's row pitch is
-    only a multiple of 4 elements (the gemm_f16_ldb4 entry)."""
+    only a multiple of 4 elements (the gemm_f16_ldb4 entry). ksplits > 1: K split over that many
+    workgroups per tile, with a workspace from torch's allocator (the gemm_f16_splitk entry)."""
     lib = load()
     for name, t in (("a", a), ("b", b), ("c", c)):
         if t.dim() != 2 or t.device.type != "cuda" or t.dtype != torch.float16:
@@ -369,6 +381,13 @@ def gemm_f16(a: torch.Tensor, b: torch.Tensor, c: torch.Tensor, tile: GemmTile, 
     K2, N = b.shape
     if K2 != K or tuple(c.shape) != (M, N):
         raise ValueError(f"incompatible GEMM shapes a={tuple(a.shape)} b={tuple(b.shape)} c={tuple(c.shape)}")
+    if ksplits > 1:
+        need = 4 * ksplits * M * N
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device)
+        check(lib.gemm_f16_splitk(a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K, a.stride(0), b.stride(0), c.stride(0),
+                                  ctypes.byref(tile), ksplits, ws.data_ptr(), need, _stream_ptr(a.device)),
+              "gemm_f16_splitk")
+        return
     code = (lib.gemm_f16_ldb4 if ldb4 else lib.gemm_f16)(
         a.data_ptr(), b.data_ptr(), c.data_ptr(), M, N, K,
         a.stride(0), b.stride(0), c.stride(0), ctypes.byref(tile), _stream_ptr(a.device),

@@ -29,20 +29,28 @@ logger = logging.getLogger(__name__)
 
 
 @functools.lru_cache(maxsize=1024)
-def _gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None, group_m: int | None):
+def _gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None,
+               group_m: int | None) -> tuple[hip_lib.GemmTile, int]:
+    """Tile and K splits of a launch with BLOCK_* hints; hints that name another tile than the one the
+    selector gives are kept (no split)."""
     try:
         bm, bn, bk, waves, gm = cfgs.choose_gemm_tile(M, N, K, hint)
+        default = hint is None or cfgs.choose_gemm_tile(M, N, K)[:4] == (bm, bn, bk, waves)
     except ValueError:
         # no built tile divides the shape: the kernel masks partial tiles (K % 8, N % 4 suffice)
         bm, bn, bk, waves, gm = cfgs.choose_gemm_tile_any(M, N, K)
-    return hip_lib.GemmTile(bm, bn, bk, waves, int(group_m) if group_m else gm)
+        default = True
+    tile, splits = cfgs.choose_gemm_splits(M, N, K, (bm, bn, bk, waves)) if default else ((bm, bn, bk, waves), 1)
+    return hip_lib.GemmTile(*tile, int(group_m) if group_m else gm), splits
 
 
 # choose_gemm_tile_any asks the library for every built tile and sorts the table: 30 us a call, three
 # times the product itself at 1000x1004x1000
 @functools.lru_cache(maxsize=1024)
-def _gemm_tile_any(M: int, N: int, K: int) -> hip_lib.GemmTile:
-    return hip_lib.GemmTile(*cfgs.choose_gemm_tile_any(M, N, K))
+def _gemm_tile_any(M: int, N: int, K: int) -> tuple[hip_lib.GemmTile, int]:
+    bm, bn, bk, waves, gm = cfgs.choose_gemm_tile_any(M, N, K)
+    tile, splits = cfgs.choose_gemm_splits(M, N, K, (bm, bn, bk, waves))
+    return hip_lib.GemmTile(*tile, gm), splits
 
 
 class _HipMatmulKernel:
@@ -83,8 +91,8 @@ class _HipMatmulKernel:
             hint = (int(kwargs["BLOCK_M"]), int(kwargs["BLOCK_N"]), int(kwargs["BLOCK_K"]))
             if kwargs.get("num_warps") is not None:
                 hint = (*hint, int(kwargs["num_warps"]))
-        tile = _gemm_tile(M, N, K, hint, kwargs.get("GROUP_M"))
-        hip_lib.gemm_f16(a, b, c, tile)
+        tile, splits = _gemm_tile(M, N, K, hint, kwargs.get("GROUP_M"))
+        hip_lib.gemm_f16(a, b, c, tile, ksplits=splits)
 
 
 _matmul_contiguous_kernel = _HipMatmulKernel()
@@ -114,18 +122,17 @@ def matmul(a: torch.Tensor, b: torch.Tensor, out: torch.Tensor | None = None) ->
     M, K = a.shape
     _, N = b.shape
     c = torch.empty((M, N), device=a.device, dtype=torch.float16) if out is None else out
-    tile = _gemm_tile_any(M, N, K)
+    tile, splits = _gemm_tile_any(M, N, K)
     if N % 8:
-        if b.data_ptr() % 16 == 0:
-            hip_lib.gemm_f16(a, b, c, tile, ldb4=True)
-            return c
-        b_rows = torch.zeros((K, N + 4), device=b.device, dtype=b.dtype)
-        b_rows[:, :N].copy_(b)
-        hip_lib.gemm_f16(a, b_rows[:, :N], c, tile)
+        if b.data_ptr() % 16:
+            b_rows = torch.zeros((K, N + 4), device=b.device, dtype=b.dtype)
+            b_rows[:, :N].copy_(b)
+            b = b_rows[:, :N]
+        hip_lib.gemm_f16(a, b, c, tile, ldb4=True, ksplits=splits)
         return c
     if not c.is_contiguous():
         raise ValueError("out must be contiguous row-major")
-    hip_lib.gemm_f16(a, b, c, tile)
+    hip_lib.gemm_f16(a, b, c, tile, ksplits=splits)
     return c
 
 

@@ -200,6 +200,15 @@ int gemm_f16(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_
 int gemm_f16_ldb4(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K,
                   int64_t lda, int64_t ldb, int64_t ldc, const gemm_tile* tile, void* stream);
 
+/* gemm_f16_ldb4 with K split over ksplits workgroups per tile (fewer when K has fewer slabs): fp32 partial
+ * products in the caller's workspace (gemm_f16_workspace_bytes), summed in split order by a second
+ * launch. For products of few tiles and a long K. Built for the 64x64x32 and 128x64x32 tiles with 8
+ * waves; FA_ENOTSUP otherwise. ksplits 1 needs no workspace. */
+int gemm_f16_splitk(const void* a, const void* b, void* c, int32_t M, int32_t N, int32_t K,
+                    int64_t lda, int64_t ldb, int64_t ldc, const gemm_tile* tile, int32_t ksplits,
+                    void* workspace, int64_t workspace_bytes, void* stream);
+int64_t gemm_f16_workspace_bytes(int32_t M, int32_t N, int32_t ksplits);
+
 int gemm_f16_supported(const gemm_tile* tile);
 
 /* Resources of one built kernel: op 0 = attention (variant, dtype, D, tile; the kernel that tile

@@ -110,6 +110,56 @@ def test_gemm_rows_of_b_on_8_byte_boundaries(gpu, shape, pad):
         torch.testing.assert_close(mma.matmul(ad, shifted), mma.matmul(ad, bd.contiguous()), rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("shape,ksplits", [((33, 4, 8), 4), ((64, 64, 64), 2), ((65, 60, 520), 3), ((130, 396, 1000), 7),
+                                           ((100, 200, 2056), 16), ((257, 1004, 4000), 5)],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else f"s{v}")
+def test_gemm_splitk(gpu, shape, ksplits):
+    """K split over the grid: one slab and more splits than slabs, a last split that is shorter, a ragged
+    K, odd slab shares of the two K groups, ragged M and N; NaN past K in A and past N in B must not
+    reach C, nothing is stored outside [M, N), and a repeat gives the same bits."""
+    M, N, K = shape
+    print(f"[gemm_tails] split-K M={M} N={N} K={K} ksplits={ksplits}", flush=True)
+    a = oracle.round_to(oracle.portable_uniform(51, (M, K), -1, 1), 0)
+    b = oracle.round_to(oracle.portable_uniform(52, (K, N), -1, 1), 0)
+    ref = oracle.gemm(a, b)
+    ad = _padded(a, K + 24, np.nan)
+    bd = _padded(b, N + 8, np.nan)
+    for tile in ((64, 64, 32, 8), (128, 64, 32, 8)):
+        first = None
+        for _ in range(2):
+            cbuf = torch.full((M, N + 8), 1234.0, dtype=torch.float16, device="cuda:0")
+            hip_lib.gemm_f16(ad, bd, cbuf[:, :N], hip_lib.GemmTile(*tile, 4), ksplits=ksplits)
+            torch.cuda.synchronize()
+            c = cbuf[:, :N].float().cpu().numpy()
+            assert np.isfinite(c).all() and bool((cbuf[:, N:] == 1234.0).all()), tile
+            assert float(np.linalg.norm(c - ref) / np.linalg.norm(ref)) <= 1e-3, tile
+            assert first is None or torch.equal(first, cbuf)
+            first = cbuf
+    with pytest.raises(ValueError, match="no split-K kernel"):
+        hip_lib.gemm_f16(ad, bd, cbuf[:, :N], hip_lib.GemmTile(128, 128, 32, 4, 4), ksplits=2)
+
+
+@pytest.mark.parametrize("shape", [(74, 608, 6216), (64, 4096, 4096), (128, 1024, 4096)], ids=lambda v: "x".join(map(str, v)))
+def test_gemm_few_tiles_long_k_takes_splits(gpu, shape):
+    """mma.matmul and the launcher split K where the time model says so; the results are those of the
+    unsplit kernel to fp32 summation order, before the one rounding to binary16."""
+    M, N, K = shape
+    g = torch.Generator(device="cuda:0").manual_seed(5)
+    a = (torch.rand(M, K, device="cuda:0", generator=g) * 2 - 1).half()
+    b = (torch.rand(K, N, device="cuda:0", generator=g) * 2 - 1).half()
+    assert mma._gemm_tile_any(M, N, K)[1] > 1
+    plain = torch.empty(M, N, device="cuda:0", dtype=torch.float16)
+    hip_lib.gemm_f16(a, b, plain, hip_lib.GemmTile(64, 64, 32, 8, 8))
+    outs = [mma.matmul(a, b)]
+    if M % 128 == 0:
+        c = torch.empty(M, N, device="cuda:0", dtype=torch.float16)
+        mma._matmul_contiguous_kernel[(1,)](a, b, c, M, N, K)
+        outs.append(c)
+    ref = a.double() @ b.double()
+    for out in outs:
+        assert float((out.double() - ref).norm() / ref.norm()) <= 1.02 * float((plain.double() - ref).norm() / ref.norm())
+
+
 def test_gemm_rejects_unaligned_tails(gpu):
     a = torch.zeros(64, 12, dtype=torch.float16, device="cuda:0")
     b = torch.zeros(12, 64, dtype=torch.float16, device="cuda:0")
