@@ -143,8 +143,18 @@ GEMM_SPLIT_US, GEMM_SPLIT_BYTES_PER_US = 2.8, 4e6
 # traffic.
 NUM_CUS = 256
 RESIDENT_DEFAULT = 2
-# Prefill-shaped sliced launches split only below this many workgroups (a quarter of the CUs).
-PREFILL_SPLIT_CUS = NUM_CUS // 4
+# Prefill-shaped sliced launches (full query tiles) split until each CU holds one workgroup, where
+# prefill_splits finds that it pays. Times in us, from one-head to 16-head grids at D = 128 (D = 64
+# and 256 scale alike): a 64-key step of a 128-row tile 0.95 (1.45 with 256 rows); a split 2.5 for
+# the merge launch, and its partials written and read back at 2.5 GB per ms. 32 blocks of 128 rows,
+# N=8192: 126 -> 37 us (81 with two splits); 128 blocks N=16384 279 -> 155, N=4096 70 -> 55; 64
+# blocks N=4096 75 -> 42; 64 blocks N=1024 (22 against 26) and 128 blocks N=2048 (36 against 41)
+# stay whole.
+PREFILL_SPLIT_CUS = NUM_CUS
+PREFILL_STEP_US = {128: 0.95, 256: 1.45}
+PREFILL_SPLIT_US = 2.5
+PREFILL_SPLIT_BYTES_PER_US = 2.5e6
+PREFILL_SPLIT_MARGIN = 1.1
 # A single sequence with two kv heads needs 128 splits to fill the resident capacity (Qwen2.5
 # B1 N32k: 18.7 us with 128 splits against 21.0 with 64, HIP-graph replay).
 MAX_SPLITS = 128
@@ -276,23 +286,33 @@ def _nearest_fa_entry(table: dict, key: str) -> dict | None:
     """The entry for `key`, else the swept bucket of the same (variant, dtype, D, causal) nearest to
     it: smallest sum of |log2| distances in B*H, M and N (ties: more work, then key order). Shapes
     between the swept sizes (the reference's B=1 H=28 pipeline cases, say) then run the tile timed on
-    their neighbours instead of the fixed preference order."""
+    their neighbours instead of the fixed preference order. Decode buckets (fewer rows than a query
+    tile: K/V streaming) and prefill buckets stand in for each other only when there is no other, and a
+    decode bucket for a prefill shape not where the other 16-bit type, whose kernels are the same, has a
+    prefill bucket (bf16 B1 H32/8 D128 N=4096 took a decode bucket's tile, 280 us against 228)."""
     entry = table.get(key)
     if entry is not None:
         return entry
     prefix, rest = key.rsplit("|", 3)[0], key.rsplit("|", 3)[1:]
     want = [int(part.lstrip("BHMN")) for part in rest]
-    best, best_rank = None, None
-    for other, ent in sorted(table.items()):
-        o_prefix, o_rest = other.rsplit("|", 3)[0], other.rsplit("|", 3)[1:]
-        if o_prefix != prefix:
-            continue
-        have = [int(part.lstrip("BHMN")) for part in o_rest]
-        dist = sum(abs(math.log2(a) - math.log2(b)) for a, b in zip(want, have))
-        rank = (dist, -have[0] * have[1] * have[2])
-        if best_rank is None or rank < best_rank:
-            best, best_rank = ent, rank
-    return best
+
+    def swept(of: str) -> list[tuple[tuple, dict]]:
+        """(rank, entry) of the buckets of one variant, dtype, head dim and causality; rank[0]: other kind."""
+        out = []
+        for other, ent in sorted(table.items()):
+            o_prefix, o_rest = other.rsplit("|", 3)[0], other.rsplit("|", 3)[1:]
+            if o_prefix == of:
+                have = [int(part.lstrip("BHMN")) for part in o_rest]
+                dist = sum(abs(math.log2(a) - math.log2(b)) for a, b in zip(want, have))
+                other_kind = (have[1] < FULL_TILE_ROWS) != (want[1] < FULL_TILE_ROWS)
+                out.append(((other_kind, dist, -have[0] * have[1] * have[2]), ent))
+        return out
+
+    own = swept(prefix)
+    if want[1] >= FULL_TILE_ROWS and own and all(rank[0] for rank, _ in own):
+        swap = ("|f16|", "|bf16|") if "|f16|" in prefix else ("|bf16|", "|f16|")
+        own += [item for item in swept(prefix.replace(*swap)) if not item[0][0]]
+    return min(own, key=lambda item: item[0], default=(None, None))[1]
 
 
 def _nearest_gemm_entry(table: dict, key: str) -> dict | None:
@@ -331,7 +351,14 @@ def _gemm_ranked_tiles(entry: dict) -> list[tuple[tuple[int, ...], int]]:
 
 
 PERSISTENT_TILE = (256, 64, 8, 9)
+FULL_TILE_ROWS = 128  # query rows from which a launch is prefill-shaped (the smaller block_m)
 KEY_GROUP_TILE = (128, 64, 8, 10)
+# Where a prefill-shaped launch splits, and a split is at most this many keys, the four-wave kernel: the
+# key groups' merge through LDS costs more than the steps it saves (bf16 B1 H1 500x5000 D128 in 20
+# splits 16.2 us against 17.7, B1 H2 128x700 in 5 12.6 against 15.4; 1024x8192 in 8 of 1024 keys: 37.7
+# against 37.3).
+SPLIT_TILE = (128, 64, 4, 5)
+SPLIT_TILE_KEYS = 512
 # A step of the key-group kernel (both groups' tiles) takes this many steps of the ping-pong kernel: it
 # has the same matrix and softmax work but fetches twice the K/V (D = 128: 2.2 us against 1.6).
 KEY_GROUP_STEP = 1.35
@@ -363,7 +390,8 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
     """Timed-table winner among candidates (the shape's bucket, else its nearest swept bucket of the
     same variant, dtype, head dim and causality), else the first candidate (preference order). Where
     that is a ping-pong or key-group tile of another bucket, key_groups_win says which of the two the
-    shape takes (a split-KV launch of few rows fills the chip by splitting: it keeps the tile)."""
+    shape takes (a split-KV launch of few rows fills the chip by splitting: it keeps the tile; one of
+    full query tiles and short splits takes SPLIT_TILE)."""
     table, key = load_tune_table()["fa"], fa_table_key(variant, dtype, D, causal, B, H, M, N)
     entry = _nearest_fa_entry(table, key)
     by_tile = {(c.block_m, c.block_n, c.waves, c.stages): c for c in reversed(candidates)}
@@ -371,9 +399,13 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
     if entry is not None:
         want = tuple(entry["tile"])
         best = next((c for t, c in reversed(by_tile.items()) if t[:len(want)] == want), best)
-    few_rows = variant == hip_lib.FA_VARIANT_SLICED and M < KEY_GROUP_TILE[0]
+    few_rows = variant == hip_lib.FA_VARIANT_SLICED and M < FULL_TILE_ROWS
     if key not in table and best.stages in (8, 9, 10) and not few_rows:
         if key_groups_win(B * H, M, N, causal):
+            if variant == hip_lib.FA_VARIANT_SLICED:
+                splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal)
+                if splits > 1 and N <= splits * SPLIT_TILE_KEYS:
+                    return by_tile.get(SPLIT_TILE, best)
             return by_tile.get(KEY_GROUP_TILE, best)
         if best.stages == 10:
             return by_tile.get(PERSISTENT_TILE, best)
@@ -398,6 +430,29 @@ def split_residency(dtype, D: int, block_m: int, block_n: int, waves: int, stage
     return max(1, min(by_regs, by_lds))
 
 
+def _prefill_us(base: int, M: int, N: int, block_m: int, causal: bool, splits: int) -> float:
+    """Modelled time of a prefill-shaped grid of base workgroups (with their splits, one or less per CU),
+    but for what does not depend on the splits. A causal block sees M keys at most, however long N is."""
+    seen = min(M, N) if causal else N
+    us = min(seen, math.ceil(N / splits)) * PREFILL_STEP_US[256 if block_m > 128 else 128] / 64
+    if splits > 1:
+        us += PREFILL_SPLIT_US + splits * base * block_m * 1024 / PREFILL_SPLIT_BYTES_PER_US
+    return us
+
+
+def prefill_splits(base: int, M: int, N: int, block_m: int, block_n: int, causal: bool) -> int:
+    """Splits that give each CU a workgroup, halved while half as many are clearly cheaper; 1 when no
+    split pays."""
+    splits = max(1, min(PREFILL_SPLIT_CUS // max(1, base), math.ceil(N / block_n) // 2, MAX_SPLITS))
+    us = _prefill_us(base, M, N, block_m, causal, splits)
+    while splits > 3:
+        half = _prefill_us(base, M, N, block_m, causal, splits // 2)
+        if half > 0.9 * us:
+            break
+        splits, us = splits // 2, half
+    return splits if us * PREFILL_SPLIT_MARGIN < _prefill_us(base, M, N, block_m, causal, 1) else 1
+
+
 @functools.lru_cache(maxsize=4096)
 def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_kv: int | None = None,
                   causal: bool = False, resident_per_cu: int = RESIDENT_DEFAULT) -> int:
@@ -407,13 +462,15 @@ def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_
     until NUM_CUS x resident_per_cu workgroups (the split kernel's resident capacity,
     split_residency) are in flight; their fp32 partials are a few rows each. Prefill-shaped grids
     (full query tiles) write partials as large as the output and read them back in the merge, so
-    they split only when they would occupy fewer than PREFILL_SPLIT_CUS CUs. Split launches of
-    decode shapes pack the query heads of a GQA group into one tile (hip_lib.pack_group), so they
+    they split up to PREFILL_SPLIT_CUS workgroups and only where that pays (prefill_splits). Split
+    launches of decode shapes pack the query heads of a GQA group into one tile (hip_lib.pack_group), so they
     count workgroups per kv head."""
     n_tiles = max(1, math.ceil(N / block_n))
     if n_tiles < 4:
         return 1
-    target = PREFILL_SPLIT_CUS if M >= block_m else NUM_CUS * max(1, resident_per_cu)
+    if M >= block_m:
+        return prefill_splits(math.ceil(M / block_m) * B * H, M, N, block_m, block_n, causal)
+    target = NUM_CUS * max(1, resident_per_cu)
 
     def splits_for(base: int) -> int:
         if base >= target:

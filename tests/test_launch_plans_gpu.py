@@ -8,9 +8,13 @@ import torch
 
 import flash_atten
 import hip_lib
+import oracle
 import tuner
+from helpers import ATOL, make_qkv, max_abs, to_device
 
 pytestmark = pytest.mark.gpu
+
+F16, BF16 = torch.float16, torch.bfloat16
 
 
 def _direct(q, k, v, causal, scale, tile, variant, lse=False, splits=1):
@@ -81,3 +85,22 @@ def test_strides_that_are_not_the_tensors_own(gpu):
     args[10] = 1 << 40  # beyond the storage: refused, as before
     with pytest.raises(RuntimeError):
         kernel[spec.grid](*args, **spec.kernel_kwargs)
+
+
+@pytest.mark.parametrize("case", [
+    (1, 2, 2, 128, 700, 128, BF16, False), (1, 4, 2, 200, 2500, 64, F16, False), (2, 2, 1, 333, 333, 128, BF16, True),
+    (1, 1, 1, 1500, 1283, 128, F16, True), (1, 4, 4, 300, 1100, 256, BF16, False), (1, 1, 1, 129, 40000, 64, BF16, False),
+], ids=lambda c: "x".join(map(str, c[:6])) + f"_c{int(c[7])}")
+def test_prefill_splits_against_the_oracle(gpu, case):
+    """Sliced prefill shapes whose keys are split over the grid, contiguous and from [B, S, H, D] storage."""
+    B, H, Hkv, M, N, D, dtype, causal = case
+    print(f"[launch_plans] prefill splits {case}", flush=True)
+    q, k, v = make_qkv(4100 + M + N, B, H, Hkv, M, N, D, dtype)
+    o_ref, lse_ref = oracle.attention(q, k, v, causal=causal)
+    qd, kd, vd = (to_device(x, dtype, "cuda:0") for x in (q, k, v))
+    o, lse = flash_atten.attention(qd, kd, vd, causal=causal, return_lse=True, variant="sliced")
+    assert max_abs(o.float().cpu().numpy(), o_ref) <= ATOL[dtype]
+    assert max_abs(lse.cpu().numpy(), lse_ref) <= 1e-3
+    qt, kt, vt = (x.transpose(1, 2).contiguous().transpose(1, 2) for x in (qd, kd, vd))
+    o = flash_atten.sdpa(qt, kt, vt, is_causal=causal, variant="sliced")
+    assert max_abs(o.float().cpu().numpy(), o_ref) <= ATOL[dtype]

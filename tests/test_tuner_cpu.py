@@ -311,6 +311,33 @@ def test_choose_splits():
     assert cfgs.choose_splits(1, 1, 64, 128, 256, 64) == 1  # too few KV tiles to split
 
 
+def test_prefill_splits():
+    """Prefill-shaped grids: one workgroup per CU at most, only where the serial steps saved outweigh the
+    partials; a causal block's steps end at its diagonal, so short-M causal launches stay whole."""
+    for B, H, M, N, block_m, causal in itertools.product((1, 3), (1, 5, 16), (128, 777, 4096), (64, 300, 2048, 40000),
+                                                         (128, 256), (False, True)):
+        base = B * H * -(-M // block_m)
+        s = cfgs.prefill_splits(base, M, N, block_m, 64, causal)
+        assert 1 <= s <= max(1, -(-N // 64) // 2) and (s == 1 or s * base <= cfgs.NUM_CUS)
+    assert cfgs.prefill_splits(32, 1024, 8192, 128, 64, False) == 8
+    assert cfgs.prefill_splits(32, 1024, 8192, 128, 64, True) == 1
+    assert cfgs.prefill_splits(128, 2048, 2048, 128, 64, True) == 1
+    assert cfgs.prefill_splits(128, 16384, 16384, 128, 64, True) == 2
+
+
+def test_prefill_tiles_of_sliced_shapes_between_the_buckets():
+    """Sliced prefill shapes take no tile of a decode bucket; short splits take the four-wave tile."""
+    def tile(dtype, D, causal, B, H, M, N):
+        t = cfgs.choose_fa_tile(hip_lib.FA_VARIANT_SLICED, dtype, D, causal, B, H, M, N,
+                                cfgs.fa_candidates(hip_lib.FA_VARIANT_SLICED, dtype, D))
+        return t.block_m, t.block_n, t.waves, t.stages
+    for dtype in (torch.float16, torch.bfloat16):
+        assert tile(dtype, 128, False, 1, 32, 3000, 3000)[3] in (8, 9)
+        assert tile(dtype, 128, False, 1, 4, 1024, 8192) == cfgs.KEY_GROUP_TILE
+        assert tile(dtype, 128, False, 1, 2, 128, 700) == cfgs.SPLIT_TILE
+    assert tile(torch.bfloat16, 128, False, 1, 32, 1, 8192)[2] == 4  # decode keeps its buckets' tiles
+
+
 def test_split_residency_follows_the_resource_table():
     # D=128 4-wave split kernels keep two workgroups per CU; the D=256 pipelined kernel (one wave
     # per SIMD) and 8-wave kernels keep one
