@@ -490,7 +490,7 @@ def gemm_cost(tile: tuple[int, int, int, int], M: int, N: int, K: int, ksplits: 
     """Modelled time (us) of a product with a tile, its K split over ksplits workgroups per tile."""
     c, lat, thr, resident = GEMM_COST[tile]
     tiles = math.ceil(M / tile[0]) * math.ceil(N / tile[1])
-    slabs = math.ceil(K / tile[2])
+    slabs = max(1, math.ceil(K / tile[2]))  # K = 0 is the launch's to refuse
     per = math.ceil(slabs / ksplits)
     parts = math.ceil(slabs / per)
     steps = math.ceil(per / GEMM_GROUPS.get(tile, 1))

@@ -280,6 +280,14 @@ def test_gemm_launch_hints_keep_the_tuned_tile():
     assert cfgs.choose_gemm_tile(8192, 8192, 8192, hint=(bm, bn, bk, warps))[:4] == (bm, bn, bk, warps)
 
 
+def test_gemm_choice_takes_empty_products():
+    """K = 0 reaches the launch, which refuses it; M = 0 and N = 0 are launches of nothing."""
+    for M, N, K in ((128, 64, 0), (64, 64, 0), (1, 4, 0), (0, 64, 64), (64, 0, 64)):
+        tile = cfgs.choose_gemm_tile_any(M, N, K)
+        assert cfgs.choose_gemm_splits(M, N, K, tile[:4]) == (tile[:4], 1)
+    assert cfgs.choose_gemm_tile(128, 64, 0)[:4] in cfgs.gemm_candidates()
+
+
 def test_cache_eviction_hint_false_without_gpu():
     assert mma._supports_contiguous_cache_eviction_hints() is torch.cuda.is_available()
 
