@@ -15,6 +15,7 @@ Tile choice never changes results, only speed.
 from __future__ import annotations
 
 import functools
+import heapq
 import json
 import math
 from dataclasses import dataclass
@@ -385,12 +386,92 @@ def key_groups_win(BH: int, M: int, N: int, causal: bool) -> bool:
     return KEY_GROUP_STEP * _serial_steps(128, 2, BH, M, N, causal) < _serial_steps(256, 1, BH, M, N, causal)
 
 
+# Time of a grid with more 256-row blocks than CUs, by simulating each kernel's schedule: us per serial
+# 64-key step (the key-group kernel: per pair of tiles) for (D, causal), fitted to 104 such grids of both
+# 16-bit types (256 to 1128 blocks, N = 2048 to 11000; error 3% at D = 128, 5% at D = 64). What the
+# simulation sees and a bucket does not: the persistent kernel's fixed sequences put heavy causal blocks
+# on the same CUs when the blocks per head do not divide them (B1 H51 causal N=4000 D128 333 us against
+# 243 of stages=8), and a last round of equal blocks that leaves most CUs idle (B1 H8 10814x11518 D64: 336
+# us against 296 of 128-row blocks, two to a CU). The choice is within 2% of the fastest of the six tiles
+# on average; the nearest bucket's was 9% slower, at worst 38%.
+GRID_STEP_US = {
+    (256, 64, 8, 9): {(64, False): 0.955, (64, True): 0.955, (128, False): 1.51, (128, True): 1.39},
+    (256, 64, 8, 8): {(64, False): 0.95, (64, True): 0.97, (128, False): 1.46, (128, True): 1.44},
+    (128, 64, 8, 10): {(64, False): 1.11, (64, True): 1.20, (128, False): 1.92, (128, True): 2.07},
+    (128, 64, 4, 6): {(64, False): 0.511, (64, True): 0.596},  # two to a CU: one at a time, in half a step's time
+}
+GRID_BLOCK_STEPS = {8: 5, 9: 3, 10: 3, 6: 3}  # what a block costs beside its steps, in steps, by stages
+GRID_F16_LEAN = 1.06  # the 4-wave kernel's f16 step in bf16 ones
+GRID_MAX_BLOCKS = 4096  # above (per simulated queue), rounds are many and the bucket's tile stays
+GRID_MODEL_MARGIN = 1.02  # the bucket's tile stays unless another is this much ahead
+GRID_SHORT_STEP_MARGIN = 1.2  # causal D = 64: blocks of few, short steps, the model's error is up to 25%
+GRID_UNTIMED_MARGIN = 1.08  # the preference order's, where no bucket of the kind was timed
+
+
+def _queue(slots: int, costs) -> float:
+    """End of a dispatch of blocks, in order, to the first free of some slots."""
+    ends = [0] * slots
+    for c in costs:
+        heapq.heapreplace(ends, ends[0] + c)
+    return max(ends)
+
+
+def _fixed_sequences(workgroups: int, costs) -> float:
+    """End of the persistent kernel's blocks: rounds over the workgroups, every second one backwards."""
+    ends = [0] * workgroups
+    for k, c in enumerate(costs):
+        r, slot = divmod(k, workgroups)
+        ends[workgroups - 1 - slot if r & 1 else slot] += c
+    return max(ends)
+
+
+@functools.lru_cache(maxsize=1024)
+def choose_full_grid_tile(f16: bool, D: int, causal: bool, BH: int, M: int, N: int,
+                          best: tuple[int, int, int, int], margin: float = GRID_MODEL_MARGIN) -> tuple[int, int, int, int]:
+    """Tile for a grid of more than NUM_CUS 256-row blocks, by the simulated schedules; best where none is
+    clearly ahead of it."""
+    if (D, causal) not in GRID_STEP_US[best]:
+        return best
+
+    def blocks(tile) -> list[int]:  # a head's blocks in dispatch order (causal: heaviest first)
+        rows, per_step = tile[0], 2 if tile[3] == 10 else 1
+        out = []
+        for i in reversed(range(math.ceil(M / rows))):
+            keys = min(N, (i + 1) * rows) if causal else N
+            out.append(GRID_BLOCK_STEPS[tile[3]] + math.ceil(math.ceil(keys / 64) / per_step))
+        return out
+
+    us = {}
+    for tile, step in GRID_STEP_US.items():
+        if (D, causal) not in step:
+            continue
+        head = blocks(tile)
+        total, slots = len(head) * BH, NUM_CUS
+        by_xcd = total % 8 == 0 and tile[3] != 10  # each XCD has its own run of blocks
+        count = total // 8 if by_xcd else total
+        if count > GRID_MAX_BLOCKS:
+            return best
+        if causal and tile[3] == 10:  # the heaviest blocks of all heads first
+            runs = [[c for c in head for _ in range(BH)]]
+        else:
+            long = head * (count // len(head) + 2)
+            runs = [long[at:at + count] for at in {x * count % len(head) for x in range(8 if by_xcd else 1)}]
+        slots = min(slots // 8 if by_xcd else slots, count)
+        schedule = _fixed_sequences if tile[3] == 9 else _queue
+        steps = max(schedule(slots, run) for run in runs)
+        us[tile] = steps * step[D, causal] * (GRID_F16_LEAN if f16 and tile[2] == 4 else 1)
+    fastest = min(us, key=us.get)
+    if causal and D == 64:
+        margin = max(margin, GRID_SHORT_STEP_MARGIN)
+    return fastest if us[fastest] * margin < us[best] else best
+
+
 def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M: int, N: int,
                    candidates: list[FaTileChoice]) -> FaTileChoice:
     """Timed-table winner among candidates (the shape's bucket, else its nearest swept bucket of the
     same variant, dtype, head dim and causality), else the first candidate (preference order). Where
-    that is a ping-pong or key-group tile of another bucket, key_groups_win says which of the two the
-    shape takes (a split-KV launch of few rows fills the chip by splitting: it keeps the tile; one of
+    that is a ping-pong or key-group tile of another bucket, key_groups_win says which of the two the shape
+    takes, and choose_full_grid_tile corrects that for more 256-row blocks than CUs (a split-KV launch of few rows fills the chip by splitting: it keeps the tile; one of
     full query tiles and short splits takes SPLIT_TILE)."""
     table, key = load_tune_table()["fa"], fa_table_key(variant, dtype, D, causal, B, H, M, N)
     entry = _nearest_fa_entry(table, key)
@@ -406,9 +487,14 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
                 splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal)
                 if splits > 1 and N <= splits * SPLIT_TILE_KEYS:
                     return by_tile.get(SPLIT_TILE, best)
-            return by_tile.get(KEY_GROUP_TILE, best)
-        if best.stages == 10:
-            return by_tile.get(PERSISTENT_TILE, best)
+            best = by_tile.get(KEY_GROUP_TILE, best)
+        elif best.stages == 10:
+            best = by_tile.get(PERSISTENT_TILE, best)
+        tile = (best.block_m, best.block_n, best.waves, best.stages)
+        if tile in GRID_STEP_US and B * H * math.ceil(M / 256) > NUM_CUS:
+            margin = GRID_MODEL_MARGIN if entry is not None else GRID_UNTIMED_MARGIN
+            f16 = "bfloat16" not in str(dtype)
+            best = by_tile.get(choose_full_grid_tile(f16, D, causal, B * H, M, N, tile, margin), best)
     return best
 
 

@@ -346,6 +346,25 @@ def test_prefill_tiles_of_sliced_shapes_between_the_buckets():
     assert tile(torch.bfloat16, 128, False, 1, 32, 1, 8192)[2] == 4  # decode keeps its buckets' tiles
 
 
+@pytest.mark.parametrize("D,causal,BH,M,N,stages", [
+    (64, False, 8, 10814, 11518, (10, 6)),    # 344 blocks: a second round of 88 on 256 CUs
+    (128, True, 51, 4000, 4000, (8,)),     # 16 blocks a head: the fixed sequences stack heavy ones
+    (128, True, 20, 5000, 5000, (10,)),
+    (128, False, 14, 8000, 8000, (8, 9)),  # 448 blocks, nearly two whole rounds
+    (64, True, 1, 65793, 65793, (8, 9, 10, 6)),  # 258 blocks, an odd count: not dealt by XCD
+])
+def test_full_grid_tiles_follow_the_schedule(D, causal, BH, M, N, stages):
+    for best in [t for t, us in cfgs.GRID_STEP_US.items() if (D, causal) in us]:
+        assert cfgs.choose_full_grid_tile(True, D, causal, BH, M, N, best)[3] in stages
+
+
+def test_full_grid_tiles_keep_the_bucket_beyond_the_model():
+    best = cfgs.PERSISTENT_TILE
+    assert cfgs.choose_full_grid_tile(True, 96, False, 64, 4096, 4096, best) == best
+    assert cfgs.choose_full_grid_tile(True, 128, True, 4096, 4096, 4096, best) == best  # too many blocks
+    assert cfgs.choose_full_grid_tile(True, 128, False, 300, 200, 0, best) in cfgs.GRID_STEP_US
+
+
 def test_split_residency_follows_the_resource_table():
     # D=128 4-wave split kernels keep two workgroups per CU; the D=256 pipelined kernel (one wave
     # per SIMD) and 8-wave kernels keep one
