@@ -331,6 +331,21 @@ def test_fa_key_groups(gpu, case):
     assert max_abs(lse, lse_ref) <= 1e-3
 
 
+@pytest.mark.parametrize("D,M,N,splits", [(64, 1, 500, 7), (128, 130, 449, 3), (128, 3, 2000, 31), (256, 40, 700, 5)])
+def test_fa_splits_keep_infinities_and_nan(gpu, D, M, N, splits):
+    """A NaN query row and infinite V elements come out of the merge as they do without splits."""
+    q, k, v = make_qkv(91 + N, 1, 2, 2, M, N, D, BF16)
+    v[:, :, N - 70:, 5] = np.inf
+    q[0, 1, M - 1] = np.nan
+    bn, stages = (32, 6) if D == 256 else (64, 7)
+    print(f"[fa_abi] special values D={D} M={M} N={N} splits={splits}", flush=True)
+    whole, _ = run_fa(q, k, v, variant=OPT, tile=(OPT, 128, bn, 4, stages), causal=False, dtype=BF16)
+    o, _ = run_fa(q, k, v, variant=SLICED, tile=(SLICED, 128, bn, 4, stages), causal=False, dtype=BF16, splits=splits)
+    for test in (np.isnan, np.isposinf):
+        assert np.array_equal(test(o), test(whole))
+    assert np.isnan(o[0, 1, M - 1]).all() and np.isposinf(o[0, 0, :, 5]).all()
+
+
 def test_fa_key_groups_fallback_and_stage_numbers(gpu):
     """A K/V row stride below D runs the 4-wave double-buffered kernel of the same rows; stages=10 on any
     other tile still means the double-buffered kernel."""
