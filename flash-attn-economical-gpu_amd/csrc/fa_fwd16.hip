@@ -128,6 +128,14 @@ struct Fwd16 {
     if (p.causal) first = min(first, (wrow0 + 1) / BN);
     return __builtin_amdgcn_readfirstlane(first - t_begin);
   }
+  // KV tiles, of the ntiles from t_begin on, that the ROWS rows from wrow0 attend to (0 without rows). A
+  // wave multiplies no tile past them: its P would be all zeros there, and 0 times an infinity or NaN
+  // in such a V row is NaN.
+  __device__ static inline int wave_tile_count(bool has_rows, int wrow0, int t_begin, int ntiles, const FwdParams& p) {
+    int n = has_rows ? ntiles : 0;
+    if (p.causal) n = min(n, (wrow0 + ROWS - 1) / BN + 1 - t_begin);
+    return __builtin_amdgcn_readfirstlane(n);
+  }
   // Key j of query i is kept when j < lim_i = N (or min(N, i + 1) causal). Each element takes a
   // sign-bit mask and a bitfield select -- vector ALU only: per-element compares would each hold a
   // scalar register pair, and the scheduler hoists all 32 of them.
@@ -555,6 +563,7 @@ struct Fwd16 {
       const int wrow0 = cur.m0 + wave * ROWS;
       const bool wave_has_rows = wrow0 < p.M;
       const int mask_from = first_masked_tile(cur.t_begin, wrow0, p);
+      const int wtiles = wave_tile_count(wave_has_rows, wrow0, cur.t_begin, ntiles, p);
       // Tile u of the current item, or tile u - ntiles of the next one (K up to the next item's
       // tile 1, V up to its tile 0), into ring slot (par + u) & 1.
       // (The next item's branch builds its descriptors there, in the two steps per item that take
@@ -652,7 +661,7 @@ struct Fwd16 {
           __builtin_amdgcn_s_setprio(0);
         };
         auto softmax_block = [&](int t) __attribute__((always_inline)) {
-          if (t < ntiles) softmax(s, pk, acc, ro, l_i, lsum, t >= mask_from, (cur.t_begin + t) * BN, wrow0, q16, g, p);
+          if (t < wtiles) softmax(s, pk, acc, ro, l_i, lsum, t >= mask_from, (cur.t_begin + t) * BN, wrow0, q16, g, p);
         };
         if (GRP == 0 && wave_has_rows) {
           qk(s, qf, kslot(0));
@@ -726,12 +735,12 @@ struct Fwd16 {
             for (int c = 0; c < kQChunks; ++c)
               if (j == min(c + 1, ntiles)) issue_q_chunk(nxt, c);
           }
-          if (wave_has_rows) {
+          if (j <= wtiles) {
             if (GRP == 0) mma_block(tog);
             else softmax_block(j - 1);
           }
           wait_vm_lds_barrier<63>();
-          if (wave_has_rows) {
+          if (j <= wtiles) {
             if (GRP == 0) softmax_block(j);
             else mma_block(tog);
           }
@@ -760,6 +769,11 @@ struct Fwd16 {
     else persistent_group<1>(p, smem, lane, wave, pid0);
   }
 
+  // SKIP: a wave multiplies no tile past its rows' last key (wave_tile_count). The test per step, which
+  // the compiler cannot take out of the loop, costs the 256-dimension kernel 1-2% (bf16 B1 H12 causal
+  // N=1973 69.5 -> 70.7 us), so there only the basic variant makes it; elsewhere it costs nothing, and
+  // the skipped products make causal grids 1-3% faster.
+  template <bool SKIP = (D <= 128)>
   __device__ static void run(const FwdParams& p) {
     __shared__ __attribute__((aligned(16))) uint16_t smem[2 * (KT_ELEMS + VT_ELEMS)];
 
@@ -826,6 +840,7 @@ struct Fwd16 {
     if (p.causal && n_end > m0 + BM) n_end = m0 + BM;
     const int t_end = (n_end + BN - 1) / BN;
     const int ntiles = t_end > t_begin ? t_end - t_begin : 0;
+    const int wtiles = wave_tile_count(wave_has_rows, wrow0, t_begin, ntiles, p);
 
     OAcc acc;
     RowOff ro;
@@ -911,7 +926,7 @@ struct Fwd16 {
         __builtin_amdgcn_s_setprio(0);
       };
       auto softmax_block = [&](int t) {
-        if (t < ntiles)
+        if (t < wtiles)
           softmax(s, pk, acc, ro, l_i, lsum, t >= mask_from, (t_begin + t) * BN, wrow0, q16, g, p);
       };
       // Group G's sequence; phases 2j and 2j+1 form iteration j. The branches on G and on
@@ -971,12 +986,12 @@ struct Fwd16 {
           issue_k(j + 1);
           issue_v(j);
           const uint16_t *kj = klane + (j & 1) * KT_ELEMS, *vp = vlane + ((j - 1) & 1) * VT_ELEMS;
-          if (wave_has_rows) {
+          if (j <= wtiles) {
             if (grp == 0) mma_block(kj, vp);
             else softmax_block(j - 1);
           }
           wait_vm_lds_barrier<63>();
-          if (wave_has_rows) {
+          if (j <= wtiles) {
             if (grp == 0) softmax_block(j);
             else mma_block(kj, vp);
           }
@@ -1016,7 +1031,7 @@ struct Fwd16 {
       auto step = [&](STile& cur, float (&mx_cur)[QT], STile& nxt, float (&mx_nxt)[QT], int u) {
         issue_k(u + 2);
         issue_v(u + 1);
-        if (wave_has_rows) {  // waves without rows still move their share of K/V
+        if (u < wtiles) {  // waves without rows or keys here still move their share of K/V
           fix_masked(cur, mx_cur, u);
           rescale(mx_cur, acc, ro, l_i, lsum, p.c);
           u32x4 pk[KC][QT];
@@ -1030,7 +1045,7 @@ struct Fwd16 {
         wait_vm_lds_barrier<0>();
       };
       auto last = [&](STile& cur, float (&mx_cur)[QT], int u) {
-        if (!wave_has_rows) return;
+        if (u >= wtiles) return;
         fix_masked(cur, mx_cur, u);
         rescale(mx_cur, acc, ro, l_i, lsum, p.c);
         u32x4 pk[KC][QT];
@@ -1062,7 +1077,7 @@ struct Fwd16 {
     for (int u = 0; u < ntiles; ++u) {
       issue_k(u + 1);
       issue_v(u + 1);
-      if (wave_has_rows) {  // waves without rows still move their share of K/V
+      if (SKIP ? u < wtiles : wave_has_rows) {  // waves without rows or keys here still move their share of K/V
         STile s;
         u32x4 pk[KC][QT];
         qk(s, qf, klane + (u & 1) * KT_ELEMS);
@@ -1203,7 +1218,7 @@ struct Fwd16 {
     }
 
     // DMA sources and ring as run(); a slot holds the K (V) tiles of both groups. Keys past N read
-    // zeros; keys of a pair's second tile past the range's end are masked.
+    // zeros; a pair's second tile past the range's end is not multiplied.
     const u32x4 krs = make_rsrc(p.k + (int64_t)b * p.sk0 + (int64_t)hk * p.sk1, (uint32_t)p.N * (uint32_t)p.sk2 * 2u);
     const u32x4 vrs = make_rsrc(p.v + (int64_t)b * p.sv0 + (int64_t)hk * p.sv1, (uint32_t)p.N * (uint32_t)p.sv2 * 2u);
     uint32_t koff, voff;
@@ -1247,10 +1262,12 @@ struct Fwd16 {
       u32x4 pk[KC][QT];
       const uint16_t* klane = smem + grp * KT_ELEMS + lane * 8;
       const uint16_t* vlane = smem + 4 * KT_ELEMS + grp * VT_ELEMS + lane * 4;
-      // first step of this group whose tile needs the mask (a tile past the range needs it too)
+      // first step of this group whose tile needs the mask
       int first = n_end / BN;
       if (p.causal) first = min(first, (wrow0 + 1) / BN);
       const int mask_from = __builtin_amdgcn_readfirstlane(max(first - t_begin - grp + 1, 0) / 2);
+      // steps whose tile is in the range and, for some row of this wave, before the diagonal
+      const int wsteps = max(wave_tile_count(wave_has_rows, wrow0, t_begin, ntiles, p) - grp + 1, 0) / 2;
       auto mma_block = [&](uint32_t tog) __attribute__((always_inline)) {  // S = Q K_j^T, O += P_{j-1} V_{j-1}
         __builtin_amdgcn_s_setprio(1);
         qk(s, qf, klane + tog * (2 * KT_ELEMS));
@@ -1259,7 +1276,7 @@ struct Fwd16 {
         __builtin_amdgcn_s_setprio(0);
       };
       auto softmax_block = [&](int u) __attribute__((always_inline)) {
-        if (u >= nsteps) return;
+        if (u >= wsteps) return;
         const int n0 = (t_begin + 2 * u + grp) * BN;
         if (u >= mask_from) mask_tile(s, n0, wrow0, q16, g, n_end, p.causal != 0);
         float mx[QT];
@@ -1322,12 +1339,12 @@ struct Fwd16 {
       for (; j <= nsteps; ++j) {
         issue_k(j + 1);
         issue_v(j);
-        if (wave_has_rows) {
+        if (j <= wsteps) {
           if (grp == 0) mma_block(j & 1);
           else softmax_block(j - 1);
         }
         wait_vm_lds_barrier<63>();
-        if (wave_has_rows) {
+        if (j <= wsteps) {
           if (grp == 0) softmax_block(j);
           else mma_block(j & 1);
         }
@@ -1430,7 +1447,7 @@ __global__ __launch_bounds__(WAVES * 64, WAVES == 8 ? 1 : 2) void fa_basic_kerne
   else if constexpr (D <= 128)
     Fwd16<Tag, D, 4, 64, 1, false>::run(p);
   else
-    Fwd16<Tag, D, 4, 32, 0, false>::run(p);
+    Fwd16<Tag, D, 4, 32, 0, false>::template run<true>(p);
 }
 
 // Registry (stages=6: PIPE 0, stages=7: PIPE 1, stages=8: PIPE 2 and stages=9: PIPE 3 with 8 waves;

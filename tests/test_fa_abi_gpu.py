@@ -331,6 +331,37 @@ def test_fa_key_groups(gpu, case):
     assert max_abs(lse, lse_ref) <= 1e-3
 
 
+@pytest.mark.parametrize("D,tile,splits", [
+    (64, (BASIC, 256, 64, 8, 1), 1), (128, (BASIC, 256, 64, 8, 1), 1), (128, (BASIC, 128, 64, 4, 1), 1),
+    (256, (BASIC, 128, 64, 4, 1), 1), (128, (OPT, 256, 64, 8, 8), 1), (128, (OPT, 128, 64, 8, 10), 1),
+    (128, (SLICED, 128, 64, 8, 10), 3), (64, (SLICED, 128, 64, 8, 10), 5), (128, (SLICED, 256, 64, 8, 9), 3),
+], ids=lambda x: "x".join(map(str, x[1:])) if isinstance(x, tuple) else str(x))
+def test_fa_values_past_the_diagonal_reach_no_row(gpu, D, tile, splits):
+    """Causal: a wave of 32 rows multiplies no tile past its last row's, so an infinity or NaN in V rows
+    that none of its rows attends to leaves its output as it is, bit for bit."""
+    M = 700
+    print(f"[fa_abi] past the diagonal D={D} {tile} splits={splits}", flush=True)
+    q, k, v = make_qkv(31 + D, 1, 2, 2, M, M, D, F16)
+    clean, _ = run_fa(q, k, v, variant=tile[0], tile=tile, causal=True, splits=splits)
+    for first, bad in ((64, np.nan), (320, np.inf), (576, np.nan)):
+        dirty = v.copy()
+        dirty[:, :, first:] = bad
+        o, _ = run_fa(q, k, dirty, variant=tile[0], tile=tile, causal=True, splits=splits)
+        rows = first // 32 * 32  # whole waves before the first bad key, which starts a tile
+        assert np.array_equal(o[:, :, :rows], clean[:, :, :rows])
+
+
+@pytest.mark.parametrize("N,splits", [(449, 3), (700, 4)])
+def test_fa_key_groups_multiply_no_tile_past_a_split(gpu, N, splits):
+    """Splits of an odd number of tiles: the second group has no tile in the last step. An infinite V
+    element of a later split makes O infinite where the oracle's is, not NaN."""
+    q, k, v = make_qkv(57 + N, 1, 2, 2, 130, N, 128, F16)
+    v[:, :, N - 100:, 5] = np.inf
+    print(f"[fa_abi] past a split N={N} splits={splits}", flush=True)
+    o, _ = run_fa(q, k, v, variant=SLICED, tile=(SLICED, 128, 64, 8, 10), causal=False, splits=splits)
+    assert np.isposinf(o[..., 5]).all() and np.isfinite(np.delete(o, 5, axis=-1)).all()
+
+
 @pytest.mark.parametrize("D,M,N,splits", [(64, 1, 500, 7), (128, 130, 449, 3), (128, 3, 2000, 31), (256, 40, 700, 5)])
 def test_fa_splits_keep_infinities_and_nan(gpu, D, M, N, splits):
     """A NaN query row and infinite V elements come out of the merge as they do without splits."""
