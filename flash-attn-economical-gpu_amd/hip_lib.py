@@ -18,7 +18,7 @@ import torch
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "libfa_gfx950.so"
 RESOURCES_PATH = HERE / "kernel_resources.json"
-ABI_VERSION = 4
+ABI_VERSION = 5
 
 FA_OK, FA_EINVAL, FA_ENOTSUP, FA_EHIP, FA_EWORKSPACE = 0, 1, 2, 3, 4
 FA_DTYPE_F16, FA_DTYPE_BF16 = 0, 1
@@ -186,13 +186,13 @@ def load() -> ctypes.CDLL:
                 "(or __graft_entry__.build()); there is no non-HIP fallback"
             )
         lib = ctypes.CDLL(str(LIB_PATH))
+        version = lib.fa_abi_version()  # first: another version may lack functions looked up below
+        if version != ABI_VERSION:
+            raise FaLibraryError(f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
         for name, (restype, argtypes) in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = restype
             fn.argtypes = argtypes
-        version = lib.fa_abi_version()
-        if version != ABI_VERSION:
-            raise FaLibraryError(f"{LIB_PATH} has ABI version {version}, expected {ABI_VERSION}; rebuild it")
         _lib = lib
         return lib
 

@@ -56,6 +56,20 @@ def test_abi_version_and_struct_layout_match_the_header(tmp_path):
             assert int(out[f"{cname}.{field}"]) == getattr(cls, field).offset, f"{cname}.{field}"
 
 
+def test_library_of_another_version_is_named_as_such(tmp_path, monkeypatch):
+    """A library built before some function existed is refused for its version, with the advice to rebuild."""
+    import subprocess
+
+    src, lib = tmp_path / "old.c", tmp_path / "libold.so"
+    src.write_text(f"int fa_abi_version(void) {{ return {hip_lib.ABI_VERSION - 1}; }}\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(lib), str(src)], check=True)
+    monkeypatch.setattr(hip_lib, "LIB_PATH", lib)
+    monkeypatch.setattr(hip_lib, "_lib", None)
+    with pytest.raises(hip_lib.FaLibraryError, match=f"ABI version {hip_lib.ABI_VERSION - 1}.*rebuild"):
+        hip_lib.load()
+    assert hip_lib._lib is None
+
+
 def test_workspace_bytes_formula():
     assert hip_lib.workspace_bytes(1, 2, 100, 128, 1) == 0
     rows = 4 * 1 * 2 * 100
