@@ -32,7 +32,8 @@ logger = logging.getLogger(__name__)
 def _gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None,
                group_m: int | None) -> tuple[hip_lib.GemmTile, int]:
     """Tile and K splits of a launch with BLOCK_* hints; hints that name another tile than the one the
-    selector gives are kept (no split)."""
+    selector gives are kept (no split). Nor is a product with N % 8 == 4 split: the launch refuses it, as
+    its B rows are not 16-byte aligned, while the split-K entry would take them."""
     try:
         bm, bn, bk, waves, gm = cfgs.choose_gemm_tile(M, N, K, hint)
         default = hint is None or cfgs.choose_gemm_tile(M, N, K)[:4] == (bm, bn, bk, waves)
@@ -40,7 +41,9 @@ def _gemm_tile(M: int, N: int, K: int, hint: tuple[int, int, int] | None,
         # no built tile divides the shape: the kernel masks partial tiles (K % 8, N % 4 suffice)
         bm, bn, bk, waves, gm = cfgs.choose_gemm_tile_any(M, N, K)
         default = True
-    tile, splits = cfgs.choose_gemm_splits(M, N, K, (bm, bn, bk, waves)) if default else ((bm, bn, bk, waves), 1)
+    tile, splits = (bm, bn, bk, waves), 1
+    if default and N % 8 == 0:
+        tile, splits = cfgs.choose_gemm_splits(M, N, K, tile)
     return hip_lib.GemmTile(*tile, int(group_m) if group_m else gm), splits
 
 

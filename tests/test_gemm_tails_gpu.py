@@ -160,6 +160,19 @@ def test_gemm_few_tiles_long_k_takes_splits(gpu, shape):
         assert float((out.double() - ref).norm() / ref.norm()) <= 1.02 * float((plain.double() - ref).norm() / ref.norm())
 
 
+@pytest.mark.parametrize("shape", [(256, 1004, 1000), (74, 612, 6216), (64, 4100, 4096), (128, 1028, 4096)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_launcher_refuses_rows_of_b_on_8_byte_boundaries(gpu, shape):
+    """The launcher's B rows start on 16-byte boundaries whatever the time model would split."""
+    M, N, K = shape
+    a, b, c = (torch.zeros(s, dtype=torch.float16, device="cuda:0") for s in ((M, K), (K, N), (M, N)))
+    with pytest.raises(ValueError, match="leading dimensions"):
+        mma._matmul_contiguous_kernel[(1,)](a, b, c, M, N, K)
+    with pytest.raises(ValueError, match="leading dimensions"):
+        mma._matmul_contiguous_kernel[(1,)](a, b, c, M, N, K, BLOCK_M=64, BLOCK_N=64, BLOCK_K=32, num_warps=8)
+    assert mma.matmul(a, b).shape == (M, N)  # mma.matmul takes them
+
+
 def test_gemm_rejects_unaligned_tails(gpu):
     a = torch.zeros(64, 12, dtype=torch.float16, device="cuda:0")
     b = torch.zeros(12, 64, dtype=torch.float16, device="cuda:0")
