@@ -182,6 +182,11 @@ def stages_for(variant: int) -> int:
 
 def fa_candidates(variant: int, dtype, D: int) -> list[FaTileChoice]:
     """Built attention tiles for (variant, dtype, D), in preference order."""
+    return list(_built_fa_tiles(variant, dtype, D))
+
+
+@functools.lru_cache(maxsize=256)
+def _built_fa_tiles(variant: int, dtype, D: int) -> tuple[FaTileChoice, ...]:
     out = []
     allowed = STAGES_BY_VARIANT.get(variant, ())
     for bm, bn, waves, stages in FA_TILE_SPACE:
@@ -195,7 +200,7 @@ def fa_candidates(variant: int, dtype, D: int) -> list[FaTileChoice]:
                 variant, dtype, D, FaTileChoice(bm, bn, waves, stages, 2).to_c()):
             continue
         out.append(choice)
-    return out
+    return tuple(out)
 
 
 @functools.lru_cache(maxsize=1)
@@ -283,6 +288,28 @@ def gemm_table_key(M: int, N: int, K: int) -> str:
     return f"M{_bucket(M)}|N{_bucket(N)}|K{_bucket(K)}"
 
 
+def _split_key(key: str) -> tuple[str, list[int]]:
+    """A table key's (variant, dtype, head dim, causality) part and its sizes."""
+    prefix, *sizes = key.rsplit("|", 3)
+    return prefix, [int(part.lstrip("BHMN")) for part in sizes]
+
+
+_indexed: tuple[dict, int, dict] | None = None  # a table, its length and its index
+
+
+def _bucket_index(table: dict) -> dict[str, list]:
+    """The attention table's buckets by kind, as (sizes, their log2, entry) in key order: parsing every key
+    at every new shape took 0.1-0.6 ms."""
+    global _indexed
+    if _indexed is None or _indexed[0] is not table or _indexed[1] != len(table):
+        index: dict[str, list] = {}
+        for key, entry in sorted(table.items()):
+            prefix, sizes = _split_key(key)
+            index.setdefault(prefix, []).append((sizes, [math.log2(x) for x in sizes], entry))
+        _indexed = (table, len(table), index)
+    return _indexed[2]
+
+
 def _nearest_fa_entry(table: dict, key: str) -> dict | None:
     """The entry for `key`, else the swept bucket of the same (variant, dtype, D, causal) nearest to
     it: smallest sum of |log2| distances in B*H, M and N (ties: more work, then key order). Shapes
@@ -294,23 +321,18 @@ def _nearest_fa_entry(table: dict, key: str) -> dict | None:
     entry = table.get(key)
     if entry is not None:
         return entry
-    prefix, rest = key.rsplit("|", 3)[0], key.rsplit("|", 3)[1:]
-    want = [int(part.lstrip("BHMN")) for part in rest]
+    prefix, sizes = _split_key(key)
+    want = [math.log2(x) for x in sizes]
+    few = sizes[1] < FULL_TILE_ROWS
+    index = _bucket_index(table)
 
     def swept(of: str) -> list[tuple[tuple, dict]]:
         """(rank, entry) of the buckets of one variant, dtype, head dim and causality; rank[0]: other kind."""
-        out = []
-        for other, ent in sorted(table.items()):
-            o_prefix, o_rest = other.rsplit("|", 3)[0], other.rsplit("|", 3)[1:]
-            if o_prefix == of:
-                have = [int(part.lstrip("BHMN")) for part in o_rest]
-                dist = sum(abs(math.log2(a) - math.log2(b)) for a, b in zip(want, have))
-                other_kind = (have[1] < FULL_TILE_ROWS) != (want[1] < FULL_TILE_ROWS)
-                out.append(((other_kind, dist, -have[0] * have[1] * have[2]), ent))
-        return out
+        return [(((have[1] < FULL_TILE_ROWS) != few, sum(abs(a - b) for a, b in zip(want, logs)),
+                  -have[0] * have[1] * have[2]), ent) for have, logs, ent in index.get(of, ())]
 
     own = swept(prefix)
-    if want[1] >= FULL_TILE_ROWS and own and all(rank[0] for rank, _ in own):
+    if not few and own and all(rank[0] for rank, _ in own):
         swap = ("|f16|", "|bf16|") if "|f16|" in prefix else ("|bf16|", "|f16|")
         own += [item for item in swept(prefix.replace(*swap)) if not item[0][0]]
     return min(own, key=lambda item: item[0], default=(None, None))[1]

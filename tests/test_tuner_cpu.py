@@ -365,6 +365,17 @@ def test_full_grid_tiles_keep_the_bucket_beyond_the_model():
     assert cfgs.choose_full_grid_tile(True, 128, False, 300, 200, 0, best) in cfgs.GRID_STEP_US
 
 
+def test_a_new_length_asks_nothing_of_the_library(monkeypatch):
+    """A length not seen before: the built tiles and the parsed table are those of earlier calls."""
+    args = (hip_lib.FA_VARIANT_SLICED, torch.bfloat16, 128)
+    flash_atten._tile_for(*args, False, 1, 32, 1, 5000, {})
+    index = cfgs._bucket_index(cfgs.load_tune_table()["fa"])
+    monkeypatch.setattr(hip_lib, "fa_fwd_supported", lambda *a: pytest.fail("the library was asked again"))
+    for M, N, causal in ((1, 5001, False), (1, 70001, False), (777, 777, True), (3001, 3001, True)):
+        flash_atten._tile_for(*args, causal, 1, 32, M, N, {})
+    assert cfgs._bucket_index(cfgs.load_tune_table()["fa"]) is index
+
+
 def test_split_residency_follows_the_resource_table():
     # D=128 4-wave split kernels keep two workgroups per CU; the D=256 pipelined kernel (one wave
     # per SIMD) and 8-wave kernels keep one
