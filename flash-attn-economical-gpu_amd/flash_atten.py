@@ -165,7 +165,7 @@ class _HipAttentionKernel:
             if splits is None:
                 splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=k.shape[1], causal=causal,
                                             resident_per_cu=cfgs.split_residency(q.dtype, D, tile.block_m, tile.block_n,
-                                                                                 tile.waves, tile.stages))
+                                                                                 tile.waves, tile.stages), D=D)
             choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, max(1, splits))
             plan = (hip_lib.fwd_plan(q, k, v, o, lse, sm_scale=sm_scale, causal=causal, variant=self.variant,
                                      tile=choice.to_c()),
@@ -286,7 +286,7 @@ def sdpa(query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, *, is_caus
             splits = cfgs.choose_splits(B, H, M, N, tile.block_m, tile.block_n, H_kv=key.shape[1],
                                         causal=bool(is_causal),
                                         resident_per_cu=cfgs.split_residency(query.dtype, D, tile.block_m, tile.block_n,
-                                                                             tile.waves, tile.stages))
+                                                                             tile.waves, tile.stages), D=D)
         choice = cfgs.FaTileChoice(tile.block_m, tile.block_n, tile.waves, tile.stages, splits)
         plan = (hip_lib.fwd_plan(query, key, value, out, None, sm_scale=sm_scale, causal=bool(is_causal),
                                  variant=variant_code, tile=choice.to_c()),

@@ -145,14 +145,14 @@ GEMM_SPLIT_US, GEMM_SPLIT_BYTES_PER_US = 2.8, 4e6
 NUM_CUS = 256
 RESIDENT_DEFAULT = 2
 # Prefill-shaped sliced launches (full query tiles) split until each CU holds one workgroup, where
-# prefill_splits finds that it pays. Times in us, from one-head to 16-head grids at D = 128 (D = 64
-# and 256 scale alike): a 64-key step of a 128-row tile 0.95 (1.45 with 256 rows); a split 2.5 for
-# the merge launch, and its partials written and read back at 2.5 GB per ms. 32 blocks of 128 rows,
-# N=8192: 126 -> 37 us (81 with two splits); 128 blocks N=16384 279 -> 155, N=4096 70 -> 55; 64
-# blocks N=4096 75 -> 42; 64 blocks N=1024 (22 against 26) and 128 blocks N=2048 (36 against 41)
-# stay whole.
+# prefill_splits finds that it pays. Times in us, from one-head to 32-head grids: a 64-key step of a
+# 128-row tile by D (with 256 rows 1.5 times that); a split 2.5 for the merge launch, and its partials
+# written and read back at 2.5 GB per ms. D = 128, 32 blocks of 128 rows, N=8192: 126 -> 37 us (81 with two
+# splits); 128 blocks N=16384 279 -> 155, N=4096 70 -> 55; 64 blocks N=4096 75 -> 42; 64 blocks N=1024
+# (22 against 26) and 128 blocks N=2048 (36 against 41) stay whole. D = 256, 6 heads 288x572 25 -> 21 in
+# 4; with D = 128's step time it stayed whole.
 PREFILL_SPLIT_CUS = NUM_CUS
-PREFILL_STEP_US = {128: 0.95, 256: 1.45}
+PREFILL_STEP_US = {64: 0.55, 128: 0.95, 256: 2.6}
 PREFILL_SPLIT_US = 2.5
 PREFILL_SPLIT_BYTES_PER_US = 2.5e6
 PREFILL_SPLIT_MARGIN = 1.1
@@ -506,7 +506,7 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
     if key not in table and best.stages in (8, 9, 10) and not few_rows:
         if key_groups_win(B * H, M, N, causal):
             if variant == hip_lib.FA_VARIANT_SLICED:
-                splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal)
+                splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal, D)
                 if splits > 1 and N <= splits * SPLIT_TILE_KEYS:
                     return by_tile.get(SPLIT_TILE, best)
             best = by_tile.get(KEY_GROUP_TILE, best)
@@ -538,32 +538,36 @@ def split_residency(dtype, D: int, block_m: int, block_n: int, waves: int, stage
     return max(1, min(by_regs, by_lds))
 
 
-def _prefill_us(base: int, M: int, N: int, block_m: int, causal: bool, splits: int) -> float:
+def _prefill_us(base: int, M: int, N: int, block_m: int, causal: bool, splits: int, D: int) -> float:
     """Modelled time of a prefill-shaped grid of base workgroups (with their splits, one or less per CU),
     but for what does not depend on the splits. A causal block sees M keys at most, however long N is."""
-    seen = min(M, N) if causal else N
-    us = min(seen, math.ceil(N / splits)) * PREFILL_STEP_US[256 if block_m > 128 else 128] / 64
+    tiles = math.ceil(math.ceil(N / 64) / splits)  # of a split
+    us = min(math.ceil((min(M, N) if causal else N) / 64), tiles) * PREFILL_STEP_US[D] * (1.5 if block_m > 128 else 1)
     if splits > 1:
-        us += PREFILL_SPLIT_US + splits * base * block_m * 1024 / PREFILL_SPLIT_BYTES_PER_US
+        rows = base * M / math.ceil(M / block_m)
+        us += PREFILL_SPLIT_US + splits * rows * D * 8 / PREFILL_SPLIT_BYTES_PER_US
     return us
 
 
-def prefill_splits(base: int, M: int, N: int, block_m: int, block_n: int, causal: bool) -> int:
+def prefill_splits(base: int, M: int, N: int, block_m: int, block_n: int, causal: bool, D: int = 128) -> int:
     """Splits that give each CU a workgroup, halved while half as many are clearly cheaper; 1 when no
-    split pays."""
-    splits = max(1, min(PREFILL_SPLIT_CUS // max(1, base), math.ceil(N / block_n) // 2, MAX_SPLITS))
-    us = _prefill_us(base, M, N, block_m, causal, splits)
+    split pays. No split is left without keys."""
+    n_tiles = max(1, math.ceil(N / block_n))
+    splits = max(1, min(PREFILL_SPLIT_CUS // max(1, base), n_tiles // 2, MAX_SPLITS))
+    us = _prefill_us(base, M, N, block_m, causal, splits, D)
     while splits > 3:
-        half = _prefill_us(base, M, N, block_m, causal, splits // 2)
+        half = _prefill_us(base, M, N, block_m, causal, splits // 2, D)
         if half > 0.9 * us:
             break
         splits, us = splits // 2, half
-    return splits if us * PREFILL_SPLIT_MARGIN < _prefill_us(base, M, N, block_m, causal, 1) else 1
+    if us * PREFILL_SPLIT_MARGIN >= _prefill_us(base, M, N, block_m, causal, 1, D):
+        return 1
+    return math.ceil(n_tiles / math.ceil(n_tiles / splits))
 
 
 @functools.lru_cache(maxsize=4096)
 def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_kv: int | None = None,
-                  causal: bool = False, resident_per_cu: int = RESIDENT_DEFAULT) -> int:
+                  causal: bool = False, resident_per_cu: int = RESIDENT_DEFAULT, D: int = 128) -> int:
     """KV splits for the sliced variant, keeping at least two KV tiles per split.
 
     Decode-shaped grids (M < block_m: a few query rows per tile, K/V streaming dominates) split
@@ -577,7 +581,9 @@ def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_
     if n_tiles < 4:
         return 1
     if M >= block_m:
-        return prefill_splits(math.ceil(M / block_m) * B * H, M, N, block_m, block_n, causal)
+        if block_m > 128 and prefill_splits(math.ceil(M / 128) * B * H, M, N, 128, block_n, causal, D) == 1:
+            return 1  # the rule the tile was chosen by (choose_fa_tile)
+        return prefill_splits(math.ceil(M / block_m) * B * H, M, N, block_m, block_n, causal, D)
     target = NUM_CUS * max(1, resident_per_cu)
 
     def splits_for(base: int) -> int:

@@ -503,7 +503,7 @@ class FlashAttentionBlockDNomaskTuner(FlashAttentionTuner):
                                             int(config["num_warps"]), int(config["num_stages"]))
             config["splits"] = cfgs.choose_splits(self.B, self.H, self.M, self.N, int(config["BLOCK_M"]),
                                                   int(config["BLOCK_N"]), H_kv=self.H_kv, causal=self.causal,
-                                                  resident_per_cu=resident)
+                                                  resident_per_cu=resident, D=self.D)
         return out
 
     def _build_candidate_launch(

@@ -327,10 +327,13 @@ def test_prefill_splits():
         base = B * H * -(-M // block_m)
         s = cfgs.prefill_splits(base, M, N, block_m, 64, causal)
         assert 1 <= s <= max(1, -(-N // 64) // 2) and (s == 1 or s * base <= cfgs.NUM_CUS)
+        assert (s - 1) * -(-(-(-N // 64)) // s) < -(-N // 64) or N == 0  # the last split has keys
     assert cfgs.prefill_splits(32, 1024, 8192, 128, 64, False) == 8
     assert cfgs.prefill_splits(32, 1024, 8192, 128, 64, True) == 1
     assert cfgs.prefill_splits(128, 2048, 2048, 128, 64, True) == 1
     assert cfgs.prefill_splits(128, 16384, 16384, 128, 64, True) == 2
+    assert cfgs.prefill_splits(18, 288, 572, 128, 32, False, 256) > 1  # D = 256: a step takes longer
+    assert cfgs.choose_splits(1, 1, 328, 328, 256, 64, causal=True, D=64) == 1  # as its 128-row blocks
 
 
 def test_prefill_tiles_of_sliced_shapes_between_the_buckets():
