@@ -79,7 +79,9 @@ const fa::GemmKernelEntry* find_gemm(const gemm_tile* t) {
 // or, when the tile asks for stages 3-10, run that LDS-DMA kernel (3-5: 32x32x16 MFMA tiles, 6-10:
 // 16x16x32 ones; the stages doc of fa_tile in the header lists them; 10 is built for one tile only).
 int stages_of(int variant, const fa_tile* t) {
-  if (variant == FA_VARIANT_BASIC) return 1;
+  // basic: its tiles' own kernels, or behind the 256-row one the per-workgroup ping-pong kernel
+  if (variant == FA_VARIANT_BASIC)
+    return t != nullptr && t->stages == 8 && t->block_m == 256 && t->block_n == 64 && t->waves == 8 ? 8 : 1;
   if (t != nullptr && t->stages == 10 && t->waves == 8 && t->block_m == 128) return 10;
   return (t != nullptr && t->stages >= 3 && t->stages <= 9) ? t->stages : 2;
 }

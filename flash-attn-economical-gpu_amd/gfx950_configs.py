@@ -15,7 +15,6 @@ Tile choice never changes results, only speed.
 from __future__ import annotations
 
 import functools
-import heapq
 import json
 import math
 from dataclasses import dataclass
@@ -382,119 +381,95 @@ KEY_GROUP_TILE = (128, 64, 8, 10)
 # against 37.3).
 SPLIT_TILE = (128, 64, 4, 5)
 SPLIT_TILE_KEYS = 512
-# A step of the key-group kernel (both groups' tiles) takes this many steps of the ping-pong kernel: it
-# has the same matrix and softmax work but fetches twice the K/V (D = 128: 2.2 us against 1.6).
-KEY_GROUP_STEP = 1.35
 
-
-def _serial_steps(rows: int, tiles_per_step: int, BH: int, M: int, N: int, causal: bool) -> float:
-    """Steps until the last of BH * ceil(M / rows) blocks ends, one workgroup per CU: the longest block's,
-    or the CUs' share of all blocks' when that is more (equal blocks run in whole rounds)."""
-    blocks = math.ceil(M / rows)
-
-    def steps(i: int) -> int:
-        keys = min(N, (i + 1) * rows) if causal else N
-        return math.ceil(math.ceil(keys / 64) / tiles_per_step)
-
-    if not causal:
-        return math.ceil(BH * blocks / NUM_CUS) * steps(0)
-    return max(steps(blocks - 1), BH * sum(steps(i) for i in range(blocks)) / NUM_CUS)
-
-
-def key_groups_win(BH: int, M: int, N: int, causal: bool) -> bool:
-    """Do 128-row blocks with two key groups end before 256-row ping-pong blocks? True where the latter
-    leave CUs idle: B1 H12 causal N=4096 (192 blocks, the longest 64 steps) 94 -> 70 us, B2 H16 777x1283
-    D64 (128 blocks) 26 -> 19, B1 H28 N=1024 29 -> 22; false at B1 H12 causal N=8192 (204 against 230)."""
-    return KEY_GROUP_STEP * _serial_steps(128, 2, BH, M, N, causal) < _serial_steps(256, 1, BH, M, N, causal)
-
-
-# Time of a grid with more 256-row blocks than CUs, by simulating each kernel's schedule: us per serial
-# 64-key step (the key-group kernel: per pair of tiles) for (D, causal), fitted to 104 such grids of both
-# 16-bit types (256 to 1128 blocks, N = 2048 to 11000; error 3% at D = 128, 5% at D = 64). What the
-# simulation sees and a bucket does not: the persistent kernel's fixed sequences put heavy causal blocks
-# on the same CUs when the blocks per head do not divide them (B1 H51 causal N=4000 D128 333 us against
-# 243 of stages=8), and a last round of equal blocks that leaves most CUs idle (B1 H8 10814x11518 D64: 336
-# us against 296 of 128-row blocks, two to a CU). The choice is within 2% of the fastest of the six tiles
-# on average; the nearest bucket's was 9% slower, at worst 38%.
-GRID_STEP_US = {
-    (256, 64, 8, 9): {(64, False): 0.955, (64, True): 0.955, (128, False): 1.51, (128, True): 1.39},
-    (256, 64, 8, 8): {(64, False): 0.95, (64, True): 0.97, (128, False): 1.46, (128, True): 1.44},
-    (128, 64, 8, 10): {(64, False): 1.11, (64, True): 1.20, (128, False): 1.92, (128, True): 2.07},
-    (128, 64, 4, 6): {(64, False): 0.511, (64, True): 0.596},  # two to a CU: one at a time, in half a step's time
+# Time of a grid with each kernel: its steps by the simulated schedule (hip_lib.grid_steps) at us per serial
+# step. Per kernel the schedule's form, (tiles per step, order, {D: blocks a CU holds}), and per (D,
+# causal) the fitted us per step, launch us, steps a block costs beside its own, time of a block alone
+# on a CU in that of two sharing one, and f16's step in bf16 ones. Fitted to every kernel's times at 2700
+# shapes of both types (1 to 160 heads, 40 to 20000 rows, 5 to 4000 us; mean error 3-7%; on 700 others
+# 3-6%, at worst 30%).
+GRID_FORM = {
+    (256, 64, 8, 8): (1, hip_lib.GRID_HEAD_MAJOR, {64: 1, 128: 1}),
+    (256, 64, 8, 9): (1, hip_lib.GRID_PERSISTENT, {64: 1, 128: 1}),
+    (128, 64, 8, 10): (2, hip_lib.GRID_HEAVIEST_FIRST, {64: 1, 128: 1}),
+    (128, 64, 4, 6): (1, hip_lib.GRID_HEAD_MAJOR, {64: 4, 128: 2}),
+    (128, 64, 4, 7): (1, hip_lib.GRID_HEAD_MAJOR, {64: 2, 128: 2}),
 }
-GRID_BLOCK_STEPS = {8: 5, 9: 3, 10: 3, 6: 3}  # what a block costs beside its steps, in steps, by stages
-GRID_F16_LEAN = 1.06  # the 4-wave kernel's f16 step in bf16 ones
-GRID_MAX_BLOCKS = 4096  # above (per simulated queue), rounds are many and the bucket's tile stays
-GRID_MODEL_MARGIN = 1.02  # the bucket's tile stays unless another is this much ahead
-GRID_SHORT_STEP_MARGIN = 1.2  # causal D = 64: blocks of few, short steps, the model's error is up to 25%
-GRID_UNTIMED_MARGIN = 1.08  # the preference order's, where no bucket of the kind was timed
+GRID_STEP_US = {
+    (256, 64, 8, 8): {(64, True): (0.865, 0.6, 6.0, 1, 0.96), (64, False): (0.867, 0.2, 6.7, 1, 0.96),
+                      (128, True): (1.302, 0.0, 5.5, 1, 0.97), (128, False): (1.325, 0.0, 5.9, 1, 0.96)},
+    (256, 64, 8, 9): {(64, True): (0.876, 1.4, 5.8, 1, 0.93), (64, False): (0.892, 1.3, 6.0, 1, 0.92),
+                      (128, True): (1.263, 0.9, 5.6, 1, 0.98), (128, False): (1.315, 0.1, 6.2, 1, 0.98)},
+    (128, 64, 8, 10): {(64, True): (1.062, 0.5, 5.2, 1, 0.93), (64, False): (1.087, 1.0, 4.4, 1, 0.91),
+                       (128, True): (1.867, 0.0, 3.8, 1, 0.98), (128, False): (1.867, 0.4, 3.4, 1, 0.98)},
+    (128, 64, 4, 6): {(64, True): (0.993, 2.5, 3.0, 0.66, 1.03), (64, False): (1.070, 3.0, 2.1, 0.60, 1.02),
+                      (128, True): (1.786, 2.5, 2.6, 0.63, 1.03), (128, False): (1.809, 2.6, 2.6, 0.61, 1.04)},
+}
+# The basic variant's bodies: the tile's own (stages 1 of 256 rows is the persistent kernel), and the
+# dispatched ping-pong kernel behind the same tile (stages 8).
+GRID_BASIC_BODY = {(256, 64, 8, 1): (256, 64, 8, 9), (256, 64, 8, 8): (256, 64, 8, 8), (128, 64, 4, 1): (128, 64, 4, 7)}
+GRID_BASIC_STEP_US = {
+    (128, 64, 4, 7): {(64, True): (1.004, 2.7, 3.1, 0.69, 0.98), (64, False): (1.001, 2.5, 3.3, 0.68, 0.98),
+                      (128, True): (1.537, 1.5, 4.0, 0.71, 1.00), (128, False): (1.631, 1.8, 3.7, 0.66, 0.99)},
+}
+# A grid of blocks that are no multiple of the XCDs spreads every head over all L2s: its steps take longer.
+GRID_UNALIGNED = 1.05
+GRID_MAX_BLOCKS = 4096  # of hip_lib.grid_steps
+# What a kernel must be ahead of the table's by to displace it. The model's errors are mostly common to
+# the kernels (clocks, caches): at 700 shapes it was not fitted to, the choice is 1.5% slower than the
+# fastest of eight timed kernels on average, at worst 27% (the nearest bucket's tile with one rule for
+# key groups and one for full grids: 5.8%, at worst 65%).
+GRID_MODEL_MARGIN = 1.0  # a nearest bucket's tile: no other margin up to 1.02 did better
+GRID_BUCKET_MARGIN = 1.03  # the shape's own bucket's, and the preference order's
+GRID_UNTIMED_MARGIN = 1.15  # the persistent kernel's, where no bucket of the kind was timed
 
 
-def _queue(slots: int, costs) -> float:
-    """End of a dispatch of blocks, in order, to the first free of some slots."""
-    ends = [0] * slots
-    for c in costs:
-        heapq.heapreplace(ends, ends[0] + c)
-    return max(ends)
+def _grid_us(body: tuple[int, int, int, int], f16: bool, D: int, causal: bool, BH: int, M: int, N: int) -> float:
+    """Modelled time of a grid with a kernel; negative where the model does not reach."""
+    per_step, order, per_cu = GRID_FORM[body]
+    step, launch, block_steps, alone, f16_step = (GRID_STEP_US.get(body) or GRID_BASIC_STEP_US[body])[D, causal]
+    steps = hip_lib.grid_steps(body[0], per_step, order, per_cu[D], block_steps, alone, BH, M, N, causal)
+    blocks = math.ceil(M / body[0]) * BH
+    if steps < 0:
+        return -1.0
+    if blocks > 64 and blocks % 8:
+        steps *= GRID_UNALIGNED
+    return launch + steps * step * (f16_step if f16 else 1)
 
 
-def _fixed_sequences(workgroups: int, costs) -> float:
-    """End of the persistent kernel's blocks: rounds over the workgroups, every second one backwards."""
-    ends = [0] * workgroups
-    for k, c in enumerate(costs):
-        r, slot = divmod(k, workgroups)
-        ends[workgroups - 1 - slot if r & 1 else slot] += c
-    return max(ends)
-
-
-@functools.lru_cache(maxsize=1024)
-def choose_full_grid_tile(f16: bool, D: int, causal: bool, BH: int, M: int, N: int,
-                          best: tuple[int, int, int, int], margin: float = GRID_MODEL_MARGIN) -> tuple[int, int, int, int]:
-    """Tile for a grid of more than NUM_CUS 256-row blocks, by the simulated schedules; best where none is
-    clearly ahead of it."""
-    if (D, causal) not in GRID_STEP_US[best]:
+@functools.lru_cache(maxsize=4096)
+def choose_full_grid_tile(f16: bool, D: int, causal: bool, BH: int, M: int, N: int, best: tuple[int, int, int, int],
+                          margin: float = GRID_MODEL_MARGIN,
+                          tiles: tuple[tuple[int, int, int, int], ...] = tuple(GRID_STEP_US)) -> tuple[int, int, int, int]:
+    """Tile of a whole-grid launch by the simulated schedules, of the given ones; best where none is ahead
+    of it by the margin, or where the model does not reach."""
+    if D not in (64, 128) or BH <= 0 or M <= 0 or best not in tiles:
         return best
-
-    def blocks(tile) -> list[int]:  # a head's blocks in dispatch order (causal: heaviest first)
-        rows, per_step = tile[0], 2 if tile[3] == 10 else 1
-        out = []
-        for i in reversed(range(math.ceil(M / rows))):
-            keys = min(N, (i + 1) * rows) if causal else N
-            out.append(GRID_BLOCK_STEPS[tile[3]] + math.ceil(math.ceil(keys / 64) / per_step))
-        return out
-
-    us = {}
-    for tile, step in GRID_STEP_US.items():
-        if (D, causal) not in step:
-            continue
-        head = blocks(tile)
-        total, slots = len(head) * BH, NUM_CUS
-        by_xcd = total % 8 == 0 and tile[3] != 10  # each XCD has its own run of blocks
-        count = total // 8 if by_xcd else total
-        if count > GRID_MAX_BLOCKS:
-            return best
-        if causal and tile[3] == 10:  # the heaviest blocks of all heads first
-            runs = [[c for c in head for _ in range(BH)]]
-        else:
-            long = head * (count // len(head) + 2)
-            runs = [long[at:at + count] for at in {x * count % len(head) for x in range(8 if by_xcd else 1)}]
-        slots = min(slots // 8 if by_xcd else slots, count)
-        schedule = _fixed_sequences if tile[3] == 9 else _queue
-        steps = max(schedule(slots, run) for run in runs)
-        us[tile] = steps * step[D, causal] * (GRID_F16_LEAN if f16 and tile[2] == 4 else 1)
+    heads = GRID_MAX_BLOCKS // math.ceil(M / 128)
+    if BH > heads >= 16:  # in many rounds the kernels compare as with fewer heads, as many over the XCDs
+        BH = heads - 8 + (BH - heads) % 8
+    us = {t: _grid_us(GRID_BASIC_BODY.get(t, t), f16, D, causal, BH, M, N) for t in tiles}
+    if min(us.values()) < 0:
+        return best
     fastest = min(us, key=us.get)
-    if causal and D == 64:
-        margin = max(margin, GRID_SHORT_STEP_MARGIN)
     return fastest if us[fastest] * margin < us[best] else best
+
+
+def _near_own_corner(table: dict, key: str, BH: int, M: int, N: int) -> bool:
+    """The shape is within a sixteenth of its swept bucket's upper corner: that timing is its own."""
+    return key in table and all(16 * x > 15 * _bucket(x) for x in (BH, M, N))
 
 
 def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M: int, N: int,
                    candidates: list[FaTileChoice]) -> FaTileChoice:
     """Timed-table winner among candidates (the shape's bucket, else its nearest swept bucket of the
-    same variant, dtype, head dim and causality), else the first candidate (preference order). Where
-    that is a ping-pong or key-group tile of another bucket, key_groups_win says which of the two the shape
-    takes, and choose_full_grid_tile corrects that for more 256-row blocks than CUs (a split-KV launch of few rows fills the chip by splitting: it keeps the tile; one of
-    full query tiles and short splits takes SPLIT_TILE)."""
+    same variant, dtype, head dim and causality), else the first candidate (preference order); but for the
+    size a bucket was timed at, the kernel that the simulated schedules put ahead of it
+    (choose_full_grid_tile). A bucket spans a factor of two in each size, and a grid's rounds, its longest
+    block and the blocks that share a CU change within it: f16 D128 causal B1 H66 N=4200 in the bucket of
+    H128 N=8192 takes 422 us with its persistent kernel and 325 dispatched. Split-KV launches
+    differ: few rows fill the chip by splitting and keep the table's tile; full query tiles that split
+    (prefill_splits) take the key-group kernel, or SPLIT_TILE for short splits."""
     table, key = load_tune_table()["fa"], fa_table_key(variant, dtype, D, causal, B, H, M, N)
     entry = _nearest_fa_entry(table, key)
     by_tile = {(c.block_m, c.block_n, c.waves, c.stages): c for c in reversed(candidates)}
@@ -502,22 +477,29 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
     if entry is not None:
         want = tuple(entry["tile"])
         best = next((c for t, c in reversed(by_tile.items()) if t[:len(want)] == want), best)
-    few_rows = variant == hip_lib.FA_VARIANT_SLICED and M < FULL_TILE_ROWS
-    if key not in table and best.stages in (8, 9, 10) and not few_rows:
-        if key_groups_win(B * H, M, N, causal):
-            if variant == hip_lib.FA_VARIANT_SLICED:
-                splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal, D)
-                if splits > 1 and N <= splits * SPLIT_TILE_KEYS:
-                    return by_tile.get(SPLIT_TILE, best)
-            best = by_tile.get(KEY_GROUP_TILE, best)
-        elif best.stages == 10:
-            best = by_tile.get(PERSISTENT_TILE, best)
-        tile = (best.block_m, best.block_n, best.waves, best.stages)
-        if tile in GRID_STEP_US and B * H * math.ceil(M / 256) > NUM_CUS:
-            margin = GRID_MODEL_MARGIN if entry is not None else GRID_UNTIMED_MARGIN
-            f16 = "bfloat16" not in str(dtype)
-            best = by_tile.get(choose_full_grid_tile(f16, D, causal, B * H, M, N, tile, margin), best)
-    return best
+    if _near_own_corner(table, key, B * H, M, N):
+        return best
+    if variant == hip_lib.FA_VARIANT_SLICED:
+        if M < FULL_TILE_ROWS:
+            return best
+        splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal, D) if KEY_GROUP_TILE in by_tile else 1
+        if splits > 1:
+            return by_tile.get(SPLIT_TILE, best) if N <= splits * SPLIT_TILE_KEYS else by_tile[KEY_GROUP_TILE]
+    if variant == hip_lib.FA_VARIANT_BASIC:  # the 256-row tile has two bodies
+        if (256, 64, 8, 1) in by_tile:
+            by_tile[256, 64, 8, 8] = FaTileChoice(256, 64, 8, 8)
+        tiles = tuple(t for t in GRID_BASIC_BODY if t in by_tile)
+    else:
+        tiles = tuple(t for t in GRID_STEP_US if t in by_tile)
+    f16, tile = "bfloat16" not in str(dtype), (best.block_m, best.block_n, best.waves, best.stages)
+    if tile not in tiles:  # a kernel the model does not know (a caller's hint, a table's choice)
+        return best
+    margin = GRID_BUCKET_MARGIN if entry is None or key in table else GRID_MODEL_MARGIN
+    if entry is None:
+        others = tuple(t for t in tiles if t != PERSISTENT_TILE)
+        tile = choose_full_grid_tile(f16, D, causal, B * H, M, N, tile, margin, others)
+        tiles, margin = (tile, *(t for t in tiles if t == PERSISTENT_TILE)), GRID_UNTIMED_MARGIN
+    return by_tile.get(choose_full_grid_tile(f16, D, causal, B * H, M, N, tile, margin, tiles), best)
 
 
 @functools.lru_cache(maxsize=256)

@@ -18,11 +18,12 @@ import torch
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "libfa_gfx950.so"
 RESOURCES_PATH = HERE / "kernel_resources.json"
-ABI_VERSION = 5
+ABI_VERSION = 6
 
 FA_OK, FA_EINVAL, FA_ENOTSUP, FA_EHIP, FA_EWORKSPACE = 0, 1, 2, 3, 4
 FA_DTYPE_F16, FA_DTYPE_BF16 = 0, 1
 FA_VARIANT_BASIC, FA_VARIANT_OPT, FA_VARIANT_SLICED = 0, 1, 2
+GRID_HEAD_MAJOR, GRID_PERSISTENT, GRID_HEAVIEST_FIRST = 0, 1, 2  # fa_grid_steps orders
 
 _DTYPE_CODES = {torch.float16: FA_DTYPE_F16, torch.bfloat16: FA_DTYPE_BF16}
 
@@ -142,6 +143,7 @@ SIGNATURES = {
     ),
     "gemm_f16_workspace_bytes": (ctypes.c_int64, [ctypes.c_int32] * 3),
     "gemm_f16_supported": (ctypes.c_int, [ctypes.POINTER(GemmTile)]),
+    "fa_grid_steps": (ctypes.c_double, [ctypes.c_int32] * 4 + [ctypes.c_double] * 2 + [ctypes.c_int32] * 4),
     "fa_kernel_resources": (
         ctypes.c_int,
         [
@@ -251,6 +253,12 @@ def workspace_bytes(B: int, H: int, M: int, D: int, splits: int) -> int:
 def pack_group(H: int, H_kv: int, M: int, causal: bool, block_m: int, splits: int) -> int:
     """Query heads fa_fwd packs into one tile's rows (1 = none); see fa_fwd_pack_group."""
     return int(load().fa_fwd_pack_group(H, H_kv, M, int(bool(causal)), block_m, splits))
+
+
+def grid_steps(rows: int, tiles_per_step: int, order: int, per_cu: int, block_steps: float, alone: float, BH: int, M: int,
+               N: int, causal: bool) -> float:
+    """Steps until an attention grid's last block ends, by the schedule model of fa_grid_steps; -1 beyond it."""
+    return load().fa_grid_steps(rows, tiles_per_step, order, per_cu, block_steps, alone, BH, M, N, int(causal))
 
 
 def fa_fwd_supported(variant: int, dtype: torch.dtype, D: int, tile: FaTile) -> bool:

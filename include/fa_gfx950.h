@@ -30,7 +30,7 @@
 extern "C" {
 #endif
 
-#define FA_ABI_VERSION 5
+#define FA_ABI_VERSION 6
 
 enum {
   FA_OK = 0,
@@ -45,10 +45,14 @@ enum { FA_DTYPE_F16 = 0, FA_DTYPE_BF16 = 1 };
 /* The three reference kernels (flash_atten.py:364-368). */
 enum { FA_VARIANT_BASIC = 0, FA_VARIANT_OPT = 1, FA_VARIANT_SLICED = 2 };
 
+/* Dispatch orders of fa_grid_steps: a head's blocks one after the other (causal: heaviest first); the same
+ * order walked by one workgroup per CU (stages 9); the heaviest blocks of all heads first (stages 10). */
+enum { FA_GRID_HEAD_MAJOR = 0, FA_GRID_PERSISTENT = 1, FA_GRID_HEAVIEST_FIRST = 2 };
+
 /* One attention tile configuration. block_m = waves * rows_per_wave (rows_per_wave in {32, 64}; 16 for stages 10);
  * block_n = KV rows per LDS tile; splits = KV splits of the sliced variant (1 = no split, no merge
- * pass). stages selects the K/V pipeline of the optimized and sliced variants (basic always runs
- * stages 1):
+ * pass). stages selects the K/V pipeline of the optimized and sliced variants (basic runs
+ * stages 1, or 8 where its 256-row tile of 64 keys and 8 waves asks for it):
  *   1  the basic kernels: with 64-key tiles and 32 rows per wave the body of stages 9 (8 waves), 7 (4
  *      waves) or 6 (D = 256), each with its rules below; the other tiles keep one K/V LDS buffer,
  *      staged through registers;
@@ -210,6 +214,13 @@ int gemm_f16_splitk(const void* a, const void* b, void* c, int32_t M, int32_t N,
 int64_t gemm_f16_workspace_bytes(int32_t M, int32_t N, int32_t ksplits);
 
 int gemm_f16_supported(const gemm_tile* tile);
+
+/* Steps until the last block of an attention grid ends on an idle chip (host only, no device): blocks of
+ * `rows` query rows, steps of `tiles_per_step` 64-key tiles, block_steps of time per block beside its
+ * steps, up to per_cu (1 to 4) blocks to a CU, where a block alone on one takes `alone` times the time of
+ * two that share it. -1 for arguments out of range or more than 4096 blocks. */
+double fa_grid_steps(int32_t rows, int32_t tiles_per_step, int32_t order, int32_t per_cu, double block_steps,
+                     double alone, int32_t BH, int32_t M, int32_t N, int32_t causal);
 
 /* Resources of one built kernel: op 0 = attention (variant, dtype, D, tile; the kernel that tile
  * resolves to, before any stages=3 fallback), op 1 = GEMM (gtile; the default deep-ring kernel).

@@ -3,6 +3,7 @@ layouts, config selection, resource errors, and the resource report. Restates th
 rules (tuner.py:72-157, 252-339, 563-590, 597-734; mma.py:63-81; exceptions.py:633-757)."""
 from __future__ import annotations
 
+import functools
 import itertools
 
 import pytest
@@ -354,7 +355,7 @@ def test_prefill_tiles_of_sliced_shapes_between_the_buckets():
     (128, True, 51, 4000, 4000, (8,)),     # 16 blocks a head: the fixed sequences stack heavy ones
     (128, True, 20, 5000, 5000, (10,)),
     (128, False, 14, 8000, 8000, (8, 9)),  # 448 blocks, nearly two whole rounds
-    (64, True, 1, 65793, 65793, (8, 9, 10, 6)),  # 258 blocks, an odd count: not dealt by XCD
+    (64, True, 1, 65793, 65793, (10,)),    # 258 blocks of 256 rows, not dealt by XCD: half the serial steps
 ])
 def test_full_grid_tiles_follow_the_schedule(D, causal, BH, M, N, stages):
     for best in [t for t, us in cfgs.GRID_STEP_US.items() if (D, causal) in us]:
@@ -365,7 +366,104 @@ def test_full_grid_tiles_keep_the_bucket_beyond_the_model():
     best = cfgs.PERSISTENT_TILE
     assert cfgs.choose_full_grid_tile(True, 96, False, 64, 4096, 4096, best) == best
     assert cfgs.choose_full_grid_tile(True, 128, True, 4096, 4096, 4096, best) == best  # too many blocks
-    assert cfgs.choose_full_grid_tile(True, 128, False, 300, 200, 0, best) in cfgs.GRID_STEP_US
+    assert cfgs.choose_full_grid_tile(True, 128, True, 1, 1 << 21, 4096, best) == best  # one head alone has too many
+    # no keys: the kernel whose launch and blocks cost least
+    assert cfgs.choose_full_grid_tile(True, 128, False, 300, 200, 0, best) == (128, 64, 4, 6)
+
+
+def _reference_steps(rows, per_step, order, block_steps, BH, M, N, causal):
+    """fa_grid_steps of one block to a CU, block by block: the persistent kernel's rounds as its item order
+    deals them, else the CUs of each XCD's four engines, served in turn and in order."""
+    nb = -(-M // rows)
+    total = nb * BH
+
+    def cost(mb):
+        keys = min(N, (mb + 1) * rows) if causal else N
+        half = 0.7 if M - mb * rows <= rows // 2 else 1.0
+        return block_steps * half + -(-(-(-keys // 64)) // per_step)
+
+    def block(pid):
+        return nb - 1 - pid % nb if causal else pid % nb
+
+    if order == hip_lib.GRID_PERSISTENT:
+        G = min(total, 256)
+        by_xcd = total % 8 == 0 and G % 8 == 0
+        S, per = (G // 8, total // 8) if by_xcd else (G, total)
+        end = 0.0
+        for w in range(G):
+            x, slot = (w & 7, w >> 3) if by_xcd else (0, w)
+            ks = (r * S + (S - 1 - slot if r & 1 else slot) for r in range(-(-per // S)))
+            end = max(end, sum(cost(block(x * per + k)) for k in ks if k < per))
+        return end
+    end = 0.0
+    for x in range(8):
+        free = [[0.0] * 8 for _ in range(4)]
+        start = 0.0
+        for i, wg in enumerate(range(x, total, 8)):
+            if order == hip_lib.GRID_HEAVIEST_FIRST and causal:
+                mb = nb - 1 - wg // BH
+            else:
+                mb = block(wg % 8 * (total // 8) + wg // 8 if total % 8 == 0 else wg)
+            engine = free[i % 4]
+            cu = engine.index(min(engine))
+            start = max(start, engine[cu])
+            engine[cu] = start + cost(mb)
+            end = max(end, engine[cu])
+    return end
+
+
+@pytest.mark.parametrize("BH,M,N", [(1, 300, 300), (3, 100, 900), (8, 2048, 2048), (66, 4200, 4200), (51, 4000, 4000),
+                                    (43, 1500, 777), (2, 3103, 3103), (144, 961, 961), (64, 2048, 4096)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_grid_steps_against_a_block_by_block_reference(BH, M, N, causal):
+    """One block, less than a round, whole rounds, counts that are no multiple of the XCDs, blocks per head
+    that divide the engines' turn, a reversed second round."""
+    for rows, per_step, order in ((256, 1, hip_lib.GRID_HEAD_MAJOR), (256, 1, hip_lib.GRID_PERSISTENT),
+                                  (128, 2, hip_lib.GRID_HEAVIEST_FIRST)):
+        got = hip_lib.grid_steps(rows, per_step, order, 1, 2.5, 1.0, BH, M, N, causal)
+        assert got == pytest.approx(_reference_steps(rows, per_step, order, 2.5, BH, M, N, causal), rel=1e-12)
+
+
+def test_grid_steps_of_shared_cus_and_refusals():
+    steps = functools.partial(hip_lib.grid_steps, 128, 1, hip_lib.GRID_HEAD_MAJOR)
+    alone = steps(2, 3.0, 0.6, 16, 2048, 1024, False)  # 256 blocks, one to a CU
+    assert 0.6 * 19 * 0.95 <= alone <= 0.6 * 19 * 1.05
+    shared = steps(2, 3.0, 0.6, 32, 2048, 1024, False)  # 512, two to a CU
+    assert 19 * 0.95 <= shared <= 19 * 1.05
+    assert shared + alone * 0.9 < steps(2, 3.0, 0.6, 48, 2048, 1024, False) <= 2 * shared  # half a round more
+    assert steps(4, 3.0, 0.6, 64, 2048, 1024, False) > shared  # three and four to a CU are slower each
+    for bad in ((0, 3.0, 0.6, 1, 64, 64, False), (5, 3.0, 0.6, 1, 64, 64, False), (1, 3.0, 0.6, 0, 64, 64, False),
+                (1, 3.0, 0.6, 1, 0, 64, False), (1, 3.0, 0.6, 1, 64, -1, False), (1, 3.0, 0.6, 4097, 128, 64, False)):
+        assert steps(*bad) == -1
+
+
+@pytest.mark.parametrize("variant,dtype,D,causal,BH,M,tiles", [
+    # inside a swept bucket, off its corner: the persistent kernel stacks heavy blocks
+    (1, torch.float16, 128, True, 66, 4200, [(256, 64, 8, 8)]), (1, torch.float16, 128, True, 113, 4000, [(256, 64, 8, 8)]),
+    (1, torch.float16, 128, True, 120, 2100, [(256, 64, 8, 8)]), (1, torch.bfloat16, 128, True, 15, 9000, [(128, 64, 8, 10)]),
+    (1, torch.float16, 128, True, 128, 4096, [(256, 64, 8, 9)]),  # the corner keeps its timing
+    # many heads of few rows: a second round of key-group blocks costs more than 256-row ones
+    (1, torch.bfloat16, 64, True, 100, 268, [(256, 64, 8, 8), (128, 64, 4, 6)]),
+    (1, torch.float16, 128, True, 116, 304, [(256, 64, 8, 8)]), (2, torch.bfloat16, 128, False, 96, 157, [(256, 64, 8, 8), (128, 64, 4, 6)]),
+    # basic: 128 rows where 256 leave CUs idle, the dispatched body where the sequences stack
+    (0, torch.float16, 128, False, 4, 1024, [(128, 64, 4, 1)]), (0, torch.bfloat16, 128, True, 37, 4273, [(256, 64, 8, 8)]),
+    (0, torch.float16, 128, True, 128, 2048, [(256, 64, 8, 1)]),
+], ids=lambda v: "x".join(map(str, v[0])) if isinstance(v, list) else str(v).replace("torch.", ""))
+def test_tiles_follow_the_schedule_of_the_shape(variant, dtype, D, causal, BH, M, tiles):
+    got = cfgs.choose_fa_tile(variant, dtype, D, causal, 1, BH, M, M, cfgs.fa_candidates(variant, dtype, D))
+    assert (got.block_m, got.block_n, got.waves, got.stages) in tiles
+
+
+@pytest.mark.parametrize("variant,D,tile", [(1, 64, (128, 64, 4, 5)), (1, 128, (128, 64, 4, 3)), (2, 64, (128, 32, 4, 6)),
+                                            (0, 128, (128, 128, 4, 1)), (1, 256, (128, 32, 4, 6)), (1, 64, (256, 64, 8, 9))])
+@pytest.mark.parametrize("causal", [False, True])
+def test_a_hinted_tile_is_kept(variant, D, tile, causal):
+    """Hints that leave one tile get it, whether the schedule model knows it and its kind was timed or not."""
+    for dtype in (torch.float16, torch.bfloat16):
+        for BH, M in ((1, 129), (1, 4000), (64, 2048), (100, 300)):
+            kw = dict(zip(("BLOCK_M", "BLOCK_N", "num_warps", "num_stages"), tile))
+            got = flash_atten._tile_for(variant, dtype, D, causal, 1, BH, M, 4000, kw)
+            assert (got.block_m, got.block_n, got.waves, got.stages) == tile
 
 
 def test_a_new_length_asks_nothing_of_the_library(monkeypatch):
