@@ -113,16 +113,19 @@ class _HipAttentionKernel:
         self._check_shapes(q, k, v, o, H, M, N, D)
         _resolve_grid(grid, kwargs)
         # the strides given are the tensors' own (what a launch spec passes): no view to build or check
-        key = None
         if (args[5:9] == q.stride() and args[9:13] == k.stride() and args[13:17] == v.stride()
                 and args[17:21] == o.stride() and (not has_lse or args[21:24] == lse.stride())):
             key = (self.variant, _form(q), _form(k), _form(v), _form(o), _form(lse) if has_lse else None, sm_scale,
                    causal, kwargs.get("BLOCK_M"), kwargs.get("BLOCK_N"), kwargs.get("num_warps"),
                    kwargs.get("num_stages"))
             plan = _plans.get(key)
-            if plan is not None:
-                hip_lib.fa_fwd_planned(plan[0], q, k, v, o, lse if has_lse else None, None, q.device.index)
-                return
+            if plan is None:
+                tile = _tile_for(self.variant, q.dtype, D, causal, q.shape[0], H, M, N, kwargs)
+                plan = (hip_lib.fwd_plan(q, k, v, o, lse if has_lse else None, sm_scale=sm_scale, causal=causal,
+                                         variant=self.variant, tile=tile.to_c()),)
+                _keep_plan(key, plan)
+            hip_lib.fa_fwd_planned(plan[0], q, k, v, o, lse if has_lse else None, None, q.device.index)
+            return
         strides = [int(s) for s in args[5:24]]
         q_v = q.as_strided(q.shape, strides[0:4])
         k_v = k.as_strided(k.shape, strides[4:8])
@@ -132,9 +135,6 @@ class _HipAttentionKernel:
         tile = _tile_for(self.variant, q.dtype, D, causal, q.shape[0], H, M, N, kwargs)
         hip_lib.fa_fwd(q_v, k_v, v_v, o_v, lse_v, sm_scale=sm_scale, causal=causal, variant=self.variant,
                        tile=tile.to_c())
-        if key is not None:
-            _keep_plan(key, (hip_lib.fwd_plan(q_v, k_v, v_v, o_v, lse_v, sm_scale=sm_scale, causal=causal,
-                                              variant=self.variant, tile=tile.to_c()),))
 
     def _launch_contiguous(self, grid, args, kwargs):
         if len(args) != 9:
