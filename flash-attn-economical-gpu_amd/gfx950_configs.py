@@ -107,36 +107,42 @@ GEMM_TILE_SPACE = [
 ]
 GEMM_DEFAULT_GROUP_M = 8
 
-# Time model of a GEMM tile, (c, lat, thr, r) in us: c + steps * max(lat * ceil(tiles / (256 r)),
-# thr * tiles / 256), with steps the K slabs one K group multiplies, lat a step alone on a CU, thr a
-# step's share of a full chip and r the workgroups a CU holds. Fitted to timings of every tile at 240
-# sizes spread over M, N, K = 64 .. 8192 (mean error 5-15%). The fastest tile by the model is within
-# 3% of the fastest timed one on average; the nearest swept bucket's was 23% slower, at worst 3.9x.
+# Time model of a GEMM tile, (c, lat, thr, e) in us and steps: c + (steps + e) * hypot(lat * ceil(tiles / 256),
+# thr * tiles / 256), with steps the K slabs one K group multiplies, lat the time of a step of a round of one
+# tile per CU, thr a step's share of a full chip and e what a tile's start and its C cost, in steps. All four
+# are fitted, to timings of every tile at 500 sizes spread over M, N, K = 64 .. 8192; on 200 others the
+# mean error is 3-8%. (With the C write left to c, and rounds of a fitted number of tiles per CU, it was
+# 6-13%, and short-K products with a large C went to the 256x256 tiles: 7808x7104x64 22.0 -> 30.8 us.)
 GEMM_COST = {
-    (256, 256, 64, 8): (5.47, 1.017, 2.531, 1),
-    (256, 256, 64, 4): (7.19, 1.124, 2.720, 4),
-    (256, 256, 32, 8): (6.05, 0.545, 1.181, 4),
-    (256, 256, 32, 4): (7.12, 0.528, 1.185, 3),
-    (256, 128, 64, 8): (4.02, 0.608, 1.708, 2),
-    (128, 256, 64, 8): (3.87, 0.605, 1.599, 3),
-    (128, 128, 64, 4): (4.18, 0.448, 0.913, 2),
-    (128, 128, 32, 4): (3.87, 0.213, 0.432, 1),
-    (128, 64, 32, 4): (3.14, 0.221, 0.266, 1),
-    (64, 256, 32, 4): (3.81, 0.240, 0.391, 1),
-    (128, 128, 32, 8): (4.52, 0.342, 1.062, 2),
-    (128, 64, 32, 8): (3.61, 0.272, 0.648, 3),
-    (128, 64, 32, 16): (4.98, 0.440, 1.360, 4),
-    (64, 64, 32, 8): (3.29, 0.221, 0.362, 1),
+    (256, 256, 64, 8): (0.00, 1.014, 1.171, 5.3),
+    (256, 256, 64, 4): (1.65, 1.140, 1.335, 4.7),
+    (256, 256, 32, 8): (0.00, 0.541, 0.583, 10.8),
+    (256, 256, 32, 4): (1.39, 0.526, 0.650, 10.6),
+    (256, 128, 64, 8): (1.85, 0.619, 0.958, 3.2),
+    (128, 256, 64, 8): (1.77, 0.615, 0.914, 3.2),
+    (128, 128, 64, 4): (3.05, 0.439, 0.462, 2.2),
+    (128, 128, 32, 4): (2.93, 0.211, 0.230, 3.7),
+    (128, 64, 32, 4): (2.71, 0.218, 0.062, 1.1),
+    (64, 256, 32, 4): (2.84, 0.233, 0.199, 3.9),
+    (128, 128, 32, 8): (2.40, 0.354, 0.535, 5.2),
+    (128, 64, 32, 8): (1.91, 0.279, 0.347, 5.2),
+    (128, 64, 32, 16): (2.78, 0.474, 0.752, 3.8),
+    (64, 64, 32, 8): (2.29, 0.216, 0.141, 3.8),
 }
 GEMM_GROUPS = {(128, 128, 32, 8): 2, (128, 64, 32, 8): 2, (128, 64, 32, 16): 4, (64, 64, 32, 8): 2}  # K groups
-# Another choice than the timed one is taken when the model puts it this much ahead (its error is smaller).
-GEMM_MODEL_MARGIN = 1.15
+# Another tile than the nearest bucket's is taken when the model puts it the first margin ahead, the second
+# where that bucket is within two octaves and its timing counts for more; a split of K when it is the third.
+# Two of 685 timed sizes are then more than 2% slower than with the nearest bucket's tile alone (nine are
+# without margins), and the choice is 3.4% slower than the fastest tile on average (the bucket's alone 38%).
+GEMM_MODEL_MARGIN = 1.1
+GEMM_NEAR_MARGIN = 1.27
+GEMM_SPLIT_MARGIN = 1.15
 # K split over the grid (hip_lib.gemm_f16 ksplits): the tiles it is built for, and its second launch's time
 # (us) and partial-sum traffic (bytes per us). 74x608x6216 29.9 -> 9.2 us in 8 splits, 64x4096x4096 20.5 ->
 # 12.1 in 4; 1000x1004x1000 (256 tiles) 8.6 -> 14 in 2, which the model refuses.
 GEMM_SPLIT_TILES = ((64, 64, 32, 8), (128, 64, 32, 8))
 GEMM_SPLITS = (2, 3, 4, 6, 8, 12, 16)
-GEMM_SPLIT_US, GEMM_SPLIT_BYTES_PER_US = 2.8, 4e6
+GEMM_SPLIT_US, GEMM_SPLIT_BYTES_PER_US = 2.7, 5e6
 
 # The sliced variant splits KV until every CU holds as many workgroups as the kernel can keep
 # resident (RESIDENT_DEFAULT when its resources are unknown); splitting further only adds merge
@@ -271,6 +277,7 @@ def load_tune_table(path: Path | None = None) -> dict:
 def reset_tune_table_cache() -> None:
     global _table_cache
     _table_cache = None
+    _ranked.clear()
 
 
 def _bucket(x: int) -> int:
@@ -356,9 +363,15 @@ def _nearest_gemm_entry(table: dict, key: str) -> dict | None:
     return best
 
 
+_ranked: dict[int, tuple[dict, list]] = {}  # of the table's entries: parsing one took 40 us, three times a call
+
+
 def _gemm_ranked_tiles(entry: dict) -> list[tuple[tuple[int, ...], int]]:
     """(tile, group_m) of a GEMM table entry, fastest first: the entry's winner, then every other
     timed (tile, GROUP_M) in order of its time."""
+    known = _ranked.get(id(entry))
+    if known is not None and known[0] is entry:
+        return known[1]
     ranked = [(tuple(entry["tile"]), int(entry.get("group_m", GEMM_DEFAULT_GROUP_M)))]
     timed = {**entry.get("timed", {}), **entry.get("refined", {})}
     for name in sorted(timed, key=timed.get):
@@ -369,6 +382,7 @@ def _gemm_ranked_tiles(entry: dict) -> list[tuple[tuple[int, ...], int]]:
             continue
         if item not in ranked:
             ranked.append(item)
+    _ranked[id(entry)] = (entry, ranked)
     return ranked
 
 
@@ -584,16 +598,23 @@ def choose_splits(B: int, H: int, M: int, N: int, block_m: int, block_n: int, H_
 
 def gemm_cost(tile: tuple[int, int, int, int], M: int, N: int, K: int, ksplits: int = 1) -> float:
     """Modelled time (us) of a product with a tile, its K split over ksplits workgroups per tile."""
-    c, lat, thr, resident = GEMM_COST[tile]
+    c, lat, thr, ends = GEMM_COST[tile]
     tiles = math.ceil(M / tile[0]) * math.ceil(N / tile[1])
     slabs = max(1, math.ceil(K / tile[2]))  # K = 0 is the launch's to refuse
     per = math.ceil(slabs / ksplits)
     parts = math.ceil(slabs / per)
     steps = math.ceil(per / GEMM_GROUPS.get(tile, 1))
-    us = c + steps * max(lat * math.ceil(tiles * parts / (NUM_CUS * resident)), thr * tiles * parts / NUM_CUS)
+    us = c + (steps + ends) * math.hypot(lat * math.ceil(tiles * parts / NUM_CUS), thr * tiles * parts / NUM_CUS)
     if ksplits > 1:
         us += GEMM_SPLIT_US + parts * M * N * 8 / GEMM_SPLIT_BYTES_PER_US
     return us
+
+
+def _octaves_to_bucket(M: int, N: int, K: int) -> float:
+    """Distance of the sizes' bucket from the nearest swept one, as _nearest_gemm_entry measures it."""
+    want = [math.log2(_bucket(x)) for x in (M, N, K)]
+    return min(sum(abs(w - math.log2(int(part.lstrip("MNK")))) for w, part in zip(want, key.split("|")))
+               for key in load_tune_table()["gemm"])
 
 
 def _swept_size(M: int, N: int, K: int) -> bool:
@@ -614,7 +635,8 @@ def _by_model(choice: tuple[int, int, int, int, int], entry: dict, candidates, M
     timed = {t for t, _ in _gemm_ranked_tiles(entry)}
     best = min((t for t in candidates if t in GEMM_COST and t in timed), key=lambda t: gemm_cost(t, M, N, K),
                default=choice[:4])
-    if gemm_cost(best, M, N, K) * GEMM_MODEL_MARGIN < gemm_cost(choice[:4], M, N, K):
+    us, best_us = gemm_cost(choice[:4], M, N, K), gemm_cost(best, M, N, K)
+    if us > GEMM_NEAR_MARGIN * best_us or us > GEMM_MODEL_MARGIN * best_us and _octaves_to_bucket(M, N, K) > 2:
         return (*best, GEMM_DEFAULT_GROUP_M)
     return choice
 
@@ -624,7 +646,7 @@ def choose_gemm_splits(M: int, N: int, K: int, tile: tuple[int, int, int, int]) 
     if tile not in GEMM_COST or _runs_persistent(tile, M, N, K):
         return tile, 1
     best = min((gemm_cost(t, M, N, K, s), t, s) for t in GEMM_SPLIT_TILES for s in GEMM_SPLITS)
-    if best[0] * GEMM_MODEL_MARGIN < gemm_cost(tile, M, N, K):
+    if best[0] * GEMM_SPLIT_MARGIN < gemm_cost(tile, M, N, K):
         return best[1], best[2]
     return tile, 1
 

@@ -281,6 +281,16 @@ def test_gemm_launch_hints_keep_the_tuned_tile():
     assert cfgs.choose_gemm_tile(8192, 8192, 8192, hint=(bm, bn, bk, warps))[:4] == (bm, bn, bk, warps)
 
 
+@pytest.mark.parametrize("M,N,K,tiles", [
+    # a large C of a short K: its write is the time, the 256x256 tiles' smaller grid makes it longer
+    (7808, 7104, 64, [(128, 64, 32, 4)]), (6912, 2624, 192, [(128, 64, 32, 4)]), (7168, 4032, 96, [(128, 64, 32, 4)]),
+    (4096, 576, 2976, [(128, 64, 32, 4)]),
+])
+def test_gemm_model_keeps_small_tiles_for_large_c(M, N, K, tiles):
+    tile = cfgs.choose_gemm_tile(M, N, K)[:4]
+    assert tile in tiles and cfgs.choose_gemm_splits(M, N, K, tile) == (tile, 1)
+
+
 def test_gemm_choice_takes_empty_products():
     """K = 0 reaches the launch, which refuses it; M = 0 and N = 0 are launches of nothing."""
     for M, N, K in ((128, 64, 0), (64, 64, 0), (1, 4, 0), (0, 64, 64), (64, 0, 64)):
