@@ -250,24 +250,21 @@ struct Fwd16 {
     }
   }
 
-  // Online softmax of one score tile: masks where needed, row max, lazy rescale, then P.
-  __device__ static inline void softmax(STile& s, u32x4 (&pk)[KC][QT], OAcc& acc, RowOff& ro,
-                                        float (&l_i)[QT], floatx4 (&lsum)[QT], bool masked, int n0, int wrow0, int q16,
-                                        int g, const FwdParams& p) {
-    if (masked) mask_tile(s, n0, wrow0, q16, g, p);
-    float mx[QT];
-    tile_max(s, mx);
-    rescale(mx, acc, ro, l_i, lsum, p.c);
-    exp_pack(s, pk, ro, l_i, p.c);
-  }
-
-  // The same for a tile that needs no mask.
+  // Online softmax of one score tile that needs no mask: row max, lazy rescale, then P.
   __device__ static inline void softmax_unmasked(const STile& s, u32x4 (&pk)[KC][QT], OAcc& acc, RowOff& ro,
                                                  float (&l_i)[QT], floatx4 (&lsum)[QT], float c) {
     float mx[QT];
     tile_max(s, mx);
     rescale(mx, acc, ro, l_i, lsum, c);
     exp_pack(s, pk, ro, l_i, c);
+  }
+
+  // The same for a tile that may need one.
+  __device__ static inline void softmax(STile& s, u32x4 (&pk)[KC][QT], OAcc& acc, RowOff& ro,
+                                        float (&l_i)[QT], floatx4 (&lsum)[QT], bool masked, int n0, int wrow0, int q16,
+                                        int g, const FwdParams& p) {
+    if (masked) mask_tile(s, n0, wrow0, q16, g, p);
+    softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
   }
 
   // P = exp2(S c - m c) rounded to the input dtype and packed as the B operand of P V; the row
@@ -710,11 +707,11 @@ struct Fwd16 {
             for (; j < fast_end; ++j) {
               fast_dma();
               if (GRP == 0) mma_block(tog);
-              else softmax(s, pk, acc, ro, l_i, lsum, false, 0, wrow0, q16, g, p);
+              else softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
               phase_fence();
               wait_vm_lds_barrier<63>();
               phase_fence();
-              if (GRP == 0) softmax(s, pk, acc, ro, l_i, lsum, false, 0, wrow0, q16, g, p);
+              if (GRP == 0) softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
               else mma_block(tog);
               phase_fence();
               advance();
@@ -968,11 +965,11 @@ struct Fwd16 {
             buffer_load16_to_lds_blocks<NVW, 32>(vr, voff, vdst + tog);
             phase_fence();
             if (grp == 0) mma_block(klane + tog / 2, vlane + (KT_ELEMS - tog / 2));
-            else softmax(s, pk, acc, ro, l_i, lsum, false, 0, wrow0, q16, g, p);
+            else softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
             phase_fence();
             wait_vm_lds_barrier<63>();
             phase_fence();
-            if (grp == 0) softmax(s, pk, acc, ro, l_i, lsum, false, 0, wrow0, q16, g, p);
+            if (grp == 0) softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
             else mma_block(klane + tog / 2, vlane + (KT_ELEMS - tog / 2));
             phase_fence();
             tog = KT_ELEMS * 2 - tog;
@@ -1279,10 +1276,7 @@ struct Fwd16 {
         if (u >= wsteps) return;
         const int n0 = (t_begin + 2 * u + grp) * BN;
         if (u >= mask_from) mask_tile(s, n0, wrow0, q16, g, n_end, p.causal != 0);
-        float mx[QT];
-        tile_max(s, mx);
-        rescale(mx, acc, ro, l_i, lsum, p.c);
-        exp_pack(s, pk, ro, l_i, p.c);
+        softmax_unmasked(s, pk, acc, ro, l_i, lsum, p.c);
       };
       issue_k(0);
       wait_vm_lds_barrier<0>();

@@ -4,6 +4,7 @@
 // same simulation in Python took 0.2-0.6 ms.
 #include <algorithm>
 #include <cstdint>
+#include <exception>
 #include <functional>  // std::greater
 #include <set>
 #include <vector>
@@ -102,10 +103,8 @@ double end_persistent(int64_t n, int workgroups, const BlockAt& at, const Grid& 
   return *std::max_element(end.begin(), end.end());
 }
 
-}  // namespace
-
-extern "C" double fa_grid_steps(int32_t rows, int32_t tiles_per_step, int32_t order, int32_t per_cu, double block_steps,
-                                double alone, int32_t BH, int32_t M, int32_t N, int32_t causal) {
+double grid_steps(int rows, int tiles_per_step, int order, int per_cu, double block_steps, double alone, int BH, int M,
+                  int N, bool causal) {
   if (rows <= 0 || tiles_per_step <= 0 || per_cu < 1 || per_cu > 4 || BH <= 0 || M <= 0 || N < 0) return -1;
   Grid g;
   g.blocks_per_head = (int)(((int64_t)M + rows - 1) / rows);
@@ -142,4 +141,15 @@ extern "C" double fa_grid_steps(int32_t rows, int32_t tiles_per_step, int32_t or
       end = std::max(end, end_exclusive(n, at, g));
   }
   return end;
+}
+
+}  // namespace
+
+extern "C" double fa_grid_steps(int32_t rows, int32_t tiles_per_step, int32_t order, int32_t per_cu, double block_steps,
+                                double alone, int32_t BH, int32_t M, int32_t N, int32_t causal) {
+  try {
+    return grid_steps(rows, tiles_per_step, order, per_cu, block_steps, alone, BH, M, N, causal != 0);
+  } catch (const std::exception&) {  // out of memory: the caller's other rule
+    return -1;
+  }
 }
