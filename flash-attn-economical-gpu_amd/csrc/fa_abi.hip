@@ -75,7 +75,7 @@ const fa::GemmKernelEntry* find_gemm(const gemm_tile* t) {
   return nullptr;
 }
 
-// Pipeline of a launch: basic keeps one K/V buffer (1); optimized and sliced double-buffer K/V (2),
+// Pipeline of a launch: basic runs its own kernels (1; 8 behind its 256-row tile); optimized and sliced double-buffer K/V (2),
 // or, when the tile asks for stages 3-10, run that LDS-DMA kernel (3-5: 32x32x16 MFMA tiles, 6-10:
 // 16x16x32 ones; the stages doc of fa_tile in the header lists them; 10 is built for one tile only).
 int stages_of(int variant, const fa_tile* t) {
@@ -145,7 +145,7 @@ const fa::FaKernelEntry* resolve_fwd(int variant, int dtype, int D, const fa_til
   return e;
 }
 
-// Does the pipelined (stages=3 or 4) kernels' addressing hold for this launch? It reads one (batch,
+// Does the addressing of the LDS-DMA kernels (pipeline() >= 3) hold for this launch? It reads one (batch,
 // kv-head) row range [0, N + block_n) of K and V with 32-bit byte offsets, and its tail check needs
 // whole rows (row stride >= D).
 bool pipelined_fits(const fa_fwd_args* a, int block_n) {
@@ -401,7 +401,7 @@ int gemm_f16_supported(const gemm_tile* tile) {
   return ok();
 }
 
-// The body of gemm_f16 and gemm_f16_ldb4: `ldb_step` is what ldb must be a multiple of. The LDS-DMA
+// The body of gemm_f16, gemm_f16_ldb4 and gemm_f16_splitk: `ldb_step` is what ldb must be a multiple of. The LDS-DMA
 // loads fetch 16 bytes per lane from any 4-byte-aligned address, and the range check works per dword, so
 // B rows that start on 8-byte boundaries need no staging: their 16-byte pieces only cross a cache line
 // now and then. Against restaging B into rows of a 16-byte pitch (a fill and a copy before the product),

@@ -17,7 +17,7 @@
 //    gfx950 transposing read ds_read_b64_tr_b16: in a 16-lane group, result lane i element c is
 //    element (i & 3) of the 8-byte chunk addressed by group lane 4c + (i >> 2). Each lane of group
 //    lane L addresses key J + (L >> 2), columns d0 + 4 (L & 3); lane i then holds V[J + c][d0 + i].
-//  * stages=1 (basic) and stages=2: K and V tiles are staged HBM -> registers -> LDS with
+//  * stages=1 (the basic tiles that fa_fwd16.hip does not build) and stages=2: K and V tiles are staged HBM -> registers -> LDS with
 //    precomputed per-thread addresses (padded rows), the next tile's global loads issued before the
 //    current tile is computed; stages=1 keeps one LDS buffer (two barriers per tile), stages=2
 //    double-buffers K/V (one barrier per tile).

@@ -1147,7 +1147,8 @@ struct Fwd16 {
   // tiles); the two partial results meet through LDS at the end, so there is no workspace and no
   // second launch. What bounds the small grids it is for is the longest block's chain of steps: bf16
   // B1 H12/2 D128 causal N=4096 94 -> 70 us (740 TFLOP/s), B2 H16 D64 777x1283 26 -> 19, fp16 B1 H28
-  // D128 N=1024 29 -> 22. A step costs 1.35 ping-pong steps, so grids that fill the chip stay there.
+  // D128 N=1024 29 -> 22. A step has a ping-pong step's products and takes 1.23 (D64) to 1.43 (D128) of
+  // its time, so grids that fill the chip stay there.
   __device__ static void run_key_groups(const FwdParams& p) {
     static_assert(PIPE != 4 || (WAVES == 8 && BN == 64 && KG == 2), "two groups of four waves");
     constexpr uint32_t kPairK = 2 * KT_ELEMS * 2, kPairV = 2 * VT_ELEMS * 2;  // bytes of a ring slot
@@ -1430,8 +1431,9 @@ __global__ __launch_bounds__(WAVES * 64, (Fwd16<Tag, D, WAVES, BN, PIPE, SPLIT>:
 }
 
 // The basic variant's kernels (stages=1): the bodies above under the basic tiles. 256 rows and 8 waves run
-// the persistent ping-pong, 128 rows and 4 waves the software pipeline, D = 256 the lean pipeline on
-// 32-key tiles. The kernels they replace kept one K/V buffer, filled through registers, with two
+// the persistent ping-pong (a tile of stages=8 the dispatched one instead, whose kernel is the registry's
+// own), 128 rows and 4 waves the software pipeline, D = 256 the lean pipeline on 32-key tiles. The
+// kernels they replace kept one K/V buffer, filled through registers, with two
 // barriers per tile and 32x32x16 MFMAs: fp16 B4 H32 D128 N=8192 4.29 -> 3.41 ms, causal N=2048 209 -> 143
 // us, bf16 B2 H16 D256 N=2048 180 -> 120 us.
 template <typename Tag, int D, int WAVES, int BN, int STAGES, bool SPLIT>

@@ -50,7 +50,7 @@ VARIANT_BY_KERNEL = {
 #   9  the ping-pong kernel in a persistent grid: one workgroup per CU walks a fixed sequence of
 #      query blocks and fetches the next block's Q, K and V during the current block's last steps,
 #  10  the ping-pong schedule with both groups on the same 128 rows and alternate KV tiles.
-# The basic variant uses stages 1; optimized and sliced use 2 to 10.
+# The basic variant uses stages 1 (or 8 behind its 256-row tile); optimized and sliced use 2 to 10.
 FA_TILE_SPACE = [
     (256, 64, 8, 8),
     (128, 32, 4, 6),
