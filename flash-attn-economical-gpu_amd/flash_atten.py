@@ -47,7 +47,7 @@ def _tile_for(variant: int, dtype: torch.dtype, D: int, causal: bool, B: int, H:
 
 @functools.lru_cache(maxsize=4096)
 def _tile_for_cached(variant, dtype, D, causal, B, H, M, N, block_m, block_n, num_warps, num_stages):
-    cands = cfgs.fa_candidates(variant, dtype, D)
+    cands = cfgs.fa_launch_candidates(variant, dtype, D)
     if not cands:
         raise hip_lib.FaUnsupportedError(
             f"attention head dim D={D} with dtype {dtype} is not built for gfx950 (D in 64/128/256, fp16/bf16)"

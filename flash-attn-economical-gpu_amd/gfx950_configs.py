@@ -50,7 +50,7 @@ VARIANT_BY_KERNEL = {
 #   9  the ping-pong kernel in a persistent grid: one workgroup per CU walks a fixed sequence of
 #      query blocks and fetches the next block's Q, K and V during the current block's last steps,
 #  10  the ping-pong schedule with both groups on the same 128 rows and alternate KV tiles.
-# The basic variant uses stages 1 (or 8 behind its 256-row tile); optimized and sliced use 2 to 10.
+# The basic variant uses stages 1 (or 8, fa_launch_candidates); optimized and sliced use 2 to 10.
 FA_TILE_SPACE = [
     (256, 64, 8, 8),
     (128, 32, 4, 6),
@@ -188,6 +188,15 @@ def stages_for(variant: int) -> int:
 def fa_candidates(variant: int, dtype, D: int) -> list[FaTileChoice]:
     """Built attention tiles for (variant, dtype, D), in preference order."""
     return list(_built_fa_tiles(variant, dtype, D))
+
+
+def fa_launch_candidates(variant: int, dtype, D: int) -> list[FaTileChoice]:
+    """The tiles a launch chooses among: the built ones and, in the basic variant, the dispatched ping-pong
+    body behind its 256-row tile, as one more tile (stages 8), so that hints tell the two apart."""
+    cands = fa_candidates(variant, dtype, D)
+    if variant == hip_lib.FA_VARIANT_BASIC and FaTileChoice(256, 64, 8, 1) in cands:
+        cands.append(FaTileChoice(256, 64, 8, 8))
+    return cands
 
 
 @functools.lru_cache(maxsize=256)
@@ -499,12 +508,8 @@ def choose_fa_tile(variant: int, dtype, D: int, causal: bool, B: int, H: int, M:
         splits = prefill_splits(B * H * math.ceil(M / 128), M, N, 128, 64, causal, D) if KEY_GROUP_TILE in by_tile else 1
         if splits > 1:
             return by_tile.get(SPLIT_TILE, best) if N <= splits * SPLIT_TILE_KEYS else by_tile[KEY_GROUP_TILE]
-    if variant == hip_lib.FA_VARIANT_BASIC:  # the 256-row tile has two bodies
-        if (256, 64, 8, 1) in by_tile:
-            by_tile[256, 64, 8, 8] = FaTileChoice(256, 64, 8, 8)
-        tiles = tuple(t for t in GRID_BASIC_BODY if t in by_tile)
-    else:
-        tiles = tuple(t for t in GRID_STEP_US if t in by_tile)
+    known = GRID_BASIC_BODY if variant == hip_lib.FA_VARIANT_BASIC else GRID_STEP_US
+    tiles = tuple(t for t in known if t in by_tile)
     f16, tile = "bfloat16" not in str(dtype), (best.block_m, best.block_n, best.waves, best.stages)
     if tile not in tiles:  # a kernel the model does not know (a caller's hint, a table's choice)
         return best

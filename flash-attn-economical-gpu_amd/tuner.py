@@ -248,7 +248,7 @@ class FlashAttentionTuner(Tuner):
 
     def _candidate_configs(self, dtype: torch.dtype = torch.float16) -> list[dict[str, int | bool]]:
         """Built gfx950 tiles for this variant/dtype/D that satisfy the tune-arg hints."""
-        cands = cfgs.fa_candidates(self.variant, dtype, self.D)
+        cands = cfgs.fa_launch_candidates(self.variant, dtype, self.D)
         if not cands:
             return []
         hints = {

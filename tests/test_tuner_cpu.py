@@ -460,12 +460,13 @@ def test_grid_steps_of_shared_cus_and_refusals():
     (0, torch.float16, 128, True, 128, 2048, [(256, 64, 8, 1)]),
 ], ids=lambda v: "x".join(map(str, v[0])) if isinstance(v, list) else str(v).replace("torch.", ""))
 def test_tiles_follow_the_schedule_of_the_shape(variant, dtype, D, causal, BH, M, tiles):
-    got = cfgs.choose_fa_tile(variant, dtype, D, causal, 1, BH, M, M, cfgs.fa_candidates(variant, dtype, D))
+    got = cfgs.choose_fa_tile(variant, dtype, D, causal, 1, BH, M, M, cfgs.fa_launch_candidates(variant, dtype, D))
     assert (got.block_m, got.block_n, got.waves, got.stages) in tiles
 
 
 @pytest.mark.parametrize("variant,D,tile", [(1, 64, (128, 64, 4, 5)), (1, 128, (128, 64, 4, 3)), (2, 64, (128, 32, 4, 6)),
-                                            (0, 128, (128, 128, 4, 1)), (1, 256, (128, 32, 4, 6)), (1, 64, (256, 64, 8, 9))])
+                                            (0, 128, (128, 128, 4, 1)), (1, 256, (128, 32, 4, 6)), (1, 64, (256, 64, 8, 9)),
+                                            (0, 64, (256, 64, 8, 1)), (0, 128, (256, 64, 8, 1)), (0, 128, (256, 64, 8, 8))])
 @pytest.mark.parametrize("causal", [False, True])
 def test_a_hinted_tile_is_kept(variant, D, tile, causal):
     """Hints that leave one tile get it, whether the schedule model knows it and its kind was timed or not."""
