@@ -11,10 +11,10 @@ Same surface as the reference's `flash_atten.py` (flash_atten.py:364-389):
   * ``flash_attention(launch_spec)`` launches a spec built by the tuners and returns ``o`` or
     ``(o, lse)``; an unknown kernel name raises NameError (flash_atten.py:370-383).
 
-Variant meaning on gfx950: basic = one fixed pipeline per tile (the persistent ping-pong, the software
-pipeline or the lean one; single-buffered K/V LDS tiles where a hint asks for its tiles); optimized = the software-
-pipelined kernel (K/V rings filled by LDS-DMA, exp work of one tile under the MFMAs of the next;
-the double-buffered kernel where a tile asks for it); sliced = split-KV partials with an LSE merge
+Variant meaning on gfx950: basic = a pipeline per tile (persistent or dispatched ping-pong, the software
+pipeline or the lean one; single-buffered K/V LDS tiles where a hint asks for its tiles); optimized = every
+built pipeline (K/V rings filled by LDS-DMA in all but the double-buffered one, exp work of one tile under
+the MFMAs of another), the one timed or modelled fastest for the shape; sliced = split-KV partials with an LSE merge
 pass (the reference's "sliced" split the head dimension instead; all three compute the same
 attention).
 """
